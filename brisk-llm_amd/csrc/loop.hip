@@ -204,8 +204,8 @@ struct SpreadStage2 {
     alignas(16) float kcur[128];                 // this token's key (its cache row)
     alignas(16) float vcur[kSpreadSlice];        // this token's values of the slice
     alignas(16) float sc[kSpreadScores];         // scores, then weights: [head][position, rows padded to 8]
-    alignas(16) uint16_t vraw[2][kSpreadStage * kSpreadSlice];  // cached values of two chunks [position][dim]
-    alignas(16) uint16_t vt[2][kSpreadSlice * kVtStride];       // the same, transposed [dim][position]
+    alignas(16) uint16_t vraw[3][kSpreadStage * kSpreadSlice];  // cached values of three chunks [position][dim]
+    alignas(16) uint16_t vt[2][kSpreadSlice * kVtStride];       // two of them transposed [dim][position]
     float mx[kSpreadHpk][4];     // [head][wave]
     double red[kSpreadHpk][4];
 };
@@ -997,10 +997,13 @@ __device__ __forceinline__ bool spread_stage2(const LoopArgs& g, const AttnArgs&
     const int cw = (chains + 63) / 64, r = t - 64 * cw, nt = kThreads - 64 * cw, wave_first = r & ~63;
     const float* rope_row = a.rope != nullptr ? a.rope + static_cast<size_t>(pos) * a.rope_dim : nullptr;
     const uint8_t* vsrc = reinterpret_cast<const uint8_t*>(a.vcache + static_cast<size_t>(kv) * a.ctx * hd + d0);
-    // chunk c's cached rows of the slice (4 pieces of 16 bytes a position) into vraw[c & 1], by the staging waves
+    // chunk c's cached rows of the slice (4 pieces of 16 bytes a position) into vraw[c % 3], by the staging waves.
+    // A staging wave transposes pieces that the others copied and starts its next copies while they may
+    // still be transposing, so a chunk's copies go to a third buffer: the one whose chunk was transposed
+    // before the last barrier.
     auto issue = [&](int c) {
         const int p0 = c * kSpreadStage, np = (pos < p0 + kSpreadStage ? pos : p0 + kSpreadStage) - p0, pieces = np * 4;
-        uint8_t* dst = reinterpret_cast<uint8_t*>(s.vraw[c & 1]);
+        uint8_t* dst = reinterpret_cast<uint8_t*>(s.vraw[c % 3]);
         for (int k = 0; k * nt < pieces; ++k) {
             const int i = k * nt + r;
             if (i < pieces)
@@ -1008,12 +1011,12 @@ __device__ __forceinline__ bool spread_stage2(const LoopArgs& g, const AttnArgs&
                                                  (lds_void_ptr)(dst + (k * nt + wave_first) * 16), 16, 0, 0);
         }
     };
-    // ... transposed to [dim][position] in vt[c & 1] (each staging wave its own pieces: whole 8 x 8
-    // blocks of 8 positions by 8 dimensions in registers, the rest a half at a time); the last chunk
+    // ... transposed to [dim][position] in vt[c & 1] (whole 8 x 8 blocks of 8 positions by 8
+    // dimensions in registers, the rest a half at a time); the last chunk
     // also takes this token's values of the slice, rounded to fp16 with the bias, at position pos
     auto transpose = [&](int c) {
         const int p0 = c * kSpreadStage, np = (pos < p0 + kSpreadStage ? pos : p0 + kSpreadStage) - p0;
-        const uint16_t* raw = s.vraw[c & 1];
+        const uint16_t* raw = s.vraw[c % 3];
         uint16_t* vt = s.vt[c & 1];
         const int blocks = (np >> 3) * (kSpreadSlice / 8);
         for (int bi = r; bi < blocks; bi += nt) {
@@ -1078,13 +1081,13 @@ __device__ __forceinline__ bool spread_stage2(const LoopArgs& g, const AttnArgs&
     } else if (wave >= cw) {
         issue(0);
         if (chunks > 1) issue(1);
+        __builtin_amdgcn_s_waitcnt(0);  // landed before the barrier: a wave transposes what the others copied
     }
     if (__syncthreads_or(fail)) {
         __builtin_amdgcn_s_waitcnt(0);
         return false;
     }
     if (wave >= cw) {  // the first chunk transposed, the third requested
-        __builtin_amdgcn_s_waitcnt(0);
         transpose(0);
         if (chunks > 2) issue(2);
     }
@@ -1130,7 +1133,7 @@ __device__ __forceinline__ bool spread_stage2(const LoopArgs& g, const AttnArgs&
     pst(st, 5);
     // value sums, one (head, dimension) chain a lane, positions in order (weighted_sum_f32, :265-273),
     // chunk by chunk; while the chain waves sum chunk c, the staging waves transpose chunk c + 1 and
-    // request chunk c + 3 (into the raw buffer chunk c + 1 leaves)
+    // request chunk c + 3 (into the raw buffer chunk c left before the last barrier)
     const bool chain = t < chains;
     const int h = chain ? t / kSpreadSlice : 0, d = t - h * kSpreadSlice;
     const float* w = s.sc + h * Ls;

@@ -131,3 +131,40 @@ def test_llama_1b_beyond_the_spread_attention():
             tok = int(np.argmax(got))
         print(f"  worst per-step logit diff {worst:.3g}; {exact} of {steps} steps bit-identical", flush=True)
         o.close()
+
+
+def test_spread_attention_over_many_chunks_repeats():
+    """2600 tokens through the token loop, whose spread attention stages the cached values in chunks of
+    256 positions while earlier chunks are summed: every run of the same tokens leaves the same logits
+    and the same caches, bit for bit (a staged chunk overwritten before it was read would show up as a
+    step that differs now and then)."""
+    import ctypes as C
+    import os
+    f, cfg, table = model.load(synth.model_path("tiny-qwen3-long"))
+    n = 2600
+    prompt = synth.prompt_ids(n, cfg.vocab, seed=3)
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    os.environ["BRISK_HIP_PREFILL"] = "0"  # token by token, through the loop
+    try:
+        s = HipSession((f, cfg, table), max_context=n + 8)
+    finally:
+        del os.environ["BRISK_HIP_PREFILL"]
+    runs = []
+    with s:
+        for k in range(4):
+            print(f"[long] tiny-qwen3-long: {n} tokens through the loop, run {k}", flush=True)
+            s.rollback(0)
+            logits = s.eval(prompt)
+            caches = []
+            for layer in range(cfg.layers):
+                for value in (False, True):
+                    ptr, nbytes = s.kv_cache(layer, value)
+                    host = np.empty(nbytes // 2, np.uint16)
+                    assert hip.hipMemcpy(C.c_void_p(host.ctypes.data), C.c_void_p(ptr), nbytes, 2) == 0  # hipMemcpyDeviceToHost
+                    caches.append(host.reshape(cfg.kv_heads, -1, cfg.head_dim)[:, :n].copy())
+            runs.append((logits, caches))
+    for k in range(1, len(runs)):
+        np.testing.assert_array_equal(runs[k][0].view(np.uint32), runs[0][0].view(np.uint32))
+        for a, b in zip(runs[k][1], runs[0][1]):
+            np.testing.assert_array_equal(a, b)
