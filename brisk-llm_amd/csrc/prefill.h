@@ -80,6 +80,14 @@ inline bool pre_attn_mfma_fits(int hpk, int head_dim) {
     return hpk >= 1 && hpk <= 64 && 64 % hpk == 0 && (head_dim == 64 || head_dim == 128);
 }
 
+// The prompt attention for 64- and 128-wide heads (k_pre_attn_rows) keeps the scores of its query rows (and
+// the rows) in LDS: kAttnRowsLds bytes a workgroup at most, so contexts up to one row's worth (39k positions).
+constexpr int kAttnRowsLds = 156 << 10;
+constexpr int attn_row_floats(int L) { return ((L + 3) & ~3) + 4; }  // rows 16-byte aligned, banks staggered
+constexpr bool pre_attn_rows_fits(int head_dim, int L) {
+    return (head_dim == 64 || head_dim == 128) && (attn_row_floats(L) + 128) * 4 <= kAttnRowsLds;
+}
+
 hipError_t launch_mm(const MmArgs& g, int mode, hipStream_t s);
 // Two store GEMMs of one activation (Q and K): one launch when both are packed-plane Q4_K of one
 // width, else launch_mm of each.

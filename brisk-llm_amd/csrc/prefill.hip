@@ -1822,21 +1822,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))
 
 // The reference's attention for a block of tokens (the same arithmetic as
 // attn_exact), arranged so that no key or value is staged: a workgroup takes R
-// query rows (R / hpk tokens x the hpk query heads of kv head blockIdx.y).
+// consecutive query rows of kv head blockIdx.y's (row = token * hpk + head).
 // Scores: a lane per position holds that position's key row in registers
 // (loaded from the cache directly) and takes every row's dot_f32 against it,
 // the query read as a broadcast; so a key is read once for all R rows and the
-// only per-score work is the 16-lane dot itself.  Softmax: a row a wave.
-// Values: a lane per (pair of dimensions, rows g, g + RG, ...), each value
-// pair read straight from the cache once for all of the lane's rows; every
-// chain adds its terms in position order, as weighted_sum_f32 does.
-constexpr int kPxRows = 16;
+// only per-score work is the 16-lane dot itself.  (The queries in scalar
+// registers, by scalar loads, were slower: each group's loads are waited for
+// whole, 4.14 ms against 4.01 for a 512-token prompt of the Llama-3.2-1B shape;
+// so was a lane taking two positions, which halves the query reads but takes the
+// registers of half the waves: 70 us a layer against 51.)
+// Softmax: a row a wave.  Values: a lane per (pair of dimensions, rows g, g + RG,
+// ...), each value pair read straight from the cache once for all of the lane's
+// rows; every chain adds its terms in position order, as weighted_sum_f32 does.
+//
+// R is the launcher's choice (attn_rows): rows share each key and value read,
+// so long batches want many, but the rows' scores of every visible position live
+// in LDS (R x L floats) and a short batch needs the workgroups.  Bound by vector
+// issue (two operations a multiply-add in the reference's order): 512 tokens of
+// the Llama-3.2-1B shape 51 us a layer; 512 tokens at 2500 positions of the
+// Qwen3-1.7B shape 435 us (R = 4).
 
 // Causal attention blocks grow with their token index, and workgroups w,
 // w + kKqCus, ... share a compute unit when the grid is resident at once.  So
 // block ids are dealt heaviest first in a snake (round r of kKqCus ids takes
 // the next kKqCus blocks, reversed on odd rounds): each unit's blocks then sum
-// to about the same work.  Block k of the heavy-first order is token block
+// to about the same work.  Block k of the heavy-first order is row block
 // nx - 1 - k / ny of kv head k % ny.
 __device__ __forceinline__ void snake_block(int id, int nx, int ny, int& y, int& x) {
     const int r = id / kKqCus, c = id - r * kKqCus;
@@ -1846,37 +1856,37 @@ __device__ __forceinline__ void snake_block(int id, int nx, int ny, int& y, int&
     x = nx - 1 - kk / ny;
     y = kk - (kk / ny) * ny;
 }
-template <int HD, int R, int LMAX>
-struct PxLds {
-    alignas(16) float q[R * HD];
-    alignas(16) float sc[R * (LMAX + 4)];
-};
 
-template <int HD, int R, int LMAX>
-__global__ __launch_bounds__(kThreads) void k_pre_attn_rows(PreAttnArgs p, int ntok) {
-    __shared__ PxLds<HD, R, LMAX> s;
+template <int HD, int R>
+__global__ __launch_bounds__(kThreads) void k_pre_attn_rows(PreAttnArgs p, int ntok, int Ls) {
+    extern __shared__ __align__(16) float px_q[];  // [R][HD] queries
+    float* const px_sc = px_q + R * HD;             // [R][Ls] scores, then weights
     constexpr int PER = HD / 16, NW = HD / 8;  // dot terms a lane partial; 16-byte pieces a key row
     const AttnArgs& g = p.a;
-    const int hpk = g.heads / g.kv_heads, tpb = R / hpk;
+    const int hpk = g.heads / g.kv_heads, all = ntok * hpk;
     int kv, xb;
-    snake_block(static_cast<int>(blockIdx.x), (ntok + tpb - 1) / tpb, g.kv_heads, kv, xb);
-    const int tb0 = xb * tpb;
-    const int ntb = ntok - tb0 < tpb ? ntok - tb0 : tpb, rows = ntb * hpk;
-    const int first = p.pos0 + tb0;  // the block's first token's position
-    const int L = first + ntb;       // positions the block's last token sees
-    const int Ls = (L + 3) & ~3;
+    snake_block(static_cast<int>(blockIdx.x), (all + R - 1) / R, g.kv_heads, kv, xb);
+    const int row0 = xb * R, rows = all - row0 < R ? all - row0 : R;
+    const int tok0 = row0 / hpk, gq0 = row0 - tok0 * hpk;  // the block's first row
+    const int first = p.pos0 + tok0;                       // its token's position
+    const int L = p.pos0 + (row0 + rows - 1) / hpk + 1;    // positions the block's last row sees
+    // sliding layers: nothing before the first row's window is read (the later rows' windows start no earlier)
+    const int p_begin = g.window > 0 && first + 1 > g.window ? (first + 1 - g.window) & ~15 : 0;
     const int t = threadIdx.x, wave = t >> 6, wl = t & 63;
     exp_tab_fill();  // ordered before the softmax by the barriers between
-    for (int i = t; i < rows * HD; i += kThreads) {  // q rows: row = token * hpk + head
-        const int row = i / HD, d = i - row * HD, tt = row / hpk, gq = row - tt * hpk;
-        s.q[i] = p.q[static_cast<size_t>(tb0 + tt) * p.qstride + (kv * hpk + gq) * HD + d];
-    }
     const uint16_t* kbase = g.kcache + static_cast<size_t>(kv) * g.ctx * HD;
     const uint16_t* vbase = g.vcache + static_cast<size_t>(kv) * g.ctx * HD;
+    __shared__ int px_tok[R];  // each row's token (divided out once)
+    if (t < R) px_tok[t] = (row0 + t) / hpk;
+    for (int i = t; i < rows * (HD / 4); i += kThreads) {
+        const int r = i / (HD / 4), tt = (row0 + r) / hpk, gq = row0 + r - tt * hpk;
+        reinterpret_cast<float4*>(px_q)[i] = gld4(p.q + static_cast<size_t>(tt) * p.qstride + (kv * hpk + gq) * HD + (i - r * (HD / 4)) * 4);
+    }
     __syncthreads();
     // ---- scores: score_p = dot_f32(q, k_p) * scale, a lane per position
-    for (int p0 = 0; p0 < L; p0 += kThreads) {
-        const int pos = p0 + t;
+    const int uwave = __builtin_amdgcn_readfirstlane(wave);
+    for (int p0 = p_begin; p0 < L; p0 += kThreads) {
+        const int pos = p0 + t, wpos = p0 + uwave * 64;
         if (pos < L) {
             uint32_t kw[HD / 2];
             const uint4* krow = reinterpret_cast<const uint4*>(kbase + static_cast<size_t>(pos) * HD);
@@ -1885,59 +1895,90 @@ __global__ __launch_bounds__(kThreads) void k_pre_attn_rows(PreAttnArgs p, int n
                 const uint4 v = krow[w];
                 kw[4 * w] = v.x; kw[4 * w + 1] = v.y; kw[4 * w + 2] = v.z; kw[4 * w + 3] = v.w;
             }
-            // rows in token order: token tt sees positions 0 .. first + tt
-            for (int tt = (pos > first ? pos - first : 0); tt < ntb; ++tt) {
-                for (int gq = 0; gq < hpk; ++gq) {
-                    const int row = tt * hpk + gq;
-                    const float* q = s.q + row * HD;
-                    // the lane partials start at their first product, not at 0 + it: they
-                    // differ only by a zero's sign, which the 0 + ... of the final sum removes
-                    float lane[16];
+            // rows in token order, from the first that sees a position of this wave (a score past
+            // its row's last position is never read)
+            const int seen = wpos > first ? (wpos - first) * hpk - gq0 : 0;
+            for (int r = seen > 0 ? seen : 0; r < rows; ++r) {
+                const float* q = px_q + r * HD;
+                // the lane partials start at their first product, not at 0 + it: they
+                // differ only by a zero's sign, which the 0 + ... of the final sum removes
+                float lane[16];
 #pragma unroll
-                    for (int m = 0; m < PER; ++m) {
-                        const float4* q4 = reinterpret_cast<const float4*>(q + 16 * m);
-                        const float4 qa = q4[0], qb = q4[1], qc = q4[2], qd = q4[3];
-                        const float qv[16] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w,
-                                              qc.x, qc.y, qc.z, qc.w, qd.x, qd.y, qd.z, qd.w};
+                for (int m = 0; m < PER; ++m) {
+                    const float4* q4 = reinterpret_cast<const float4*>(q + 16 * m);
+                    const float4 qa = q4[0], qb = q4[1], qc = q4[2], qd = q4[3];
+                    const float qv[16] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w,
+                                          qc.x, qc.y, qc.z, qc.w, qd.x, qd.y, qd.z, qd.w};
 #pragma unroll
-                        for (int j = 0; j < 16; ++j) {
-                            const float pr = (j & 1) ? mul_h<true>(qv[j], kw[8 * m + (j >> 1)]) : mul_h<false>(qv[j], kw[8 * m + (j >> 1)]);
-                            lane[j] = m == 0 ? pr : lane[j] + pr;
-                        }
+                    for (int j = 0; j < 16; ++j) {
+                        const float pr = (j & 1) ? mul_h<true>(qv[j], kw[8 * m + (j >> 1)]) : mul_h<false>(qv[j], kw[8 * m + (j >> 1)]);
+                        lane[j] = m == 0 ? pr : lane[j] + pr;
                     }
-                    float sum = 0.0f;
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) sum += lane[j];
-                    s.sc[row * Ls + pos] = sum * g.scale;
                 }
+                float sum = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 16; ++j) sum += lane[j];
+                px_sc[r * Ls + pos] = sum * g.scale;
             }
         }
     }
     __syncthreads();
-    // ---- softmax, a row a wave: max, e = expf(s - max), double sum, w = e * (float)(1 / sum)
+    // ---- softmax: max, e = expf(s - max), double sum, w = e * (float)(1 / sum).
     // A sliding layer's row sees positions start .. Lr - 1 (src/model.cpp:1084-1088): the weights
     // before start are set to zero, so the value sums below add +0 until start and then the
     // same terms in the same order as from start.
-    for (int row = wave; row < rows; row += kThreads / 64) {
-        const int Lr = first + row / hpk + 1;
-        const int start = g.window > 0 && Lr > g.window ? Lr - g.window : 0;
-        float* sc = s.sc + row * Ls;
-        float m = -INFINITY;
-        for (int q = start + wl; q < Lr; q += 64) m = fmaxf(m, sc[q]);
-        m = wave_max(m);
-        double part = 0.0;
-        for (int q = start + wl; q < Lr; q += 64) {
-            const float e = ref_expf_s(sc[q] - m);
-            sc[q] = e;
-            part += static_cast<double>(e);
+    auto span = [&](int r, int& start, int& Lr) {
+        Lr = p.pos0 + px_tok[r] + 1;
+        start = g.window > 0 && Lr > g.window ? Lr - g.window : 0;
+    };
+    if constexpr (R >= 4) {  // a row a wave
+        for (int r = wave; r < rows; r += kThreads / 64) {
+            int start, Lr;
+            span(r, start, Lr);
+            float* sc = px_sc + r * Ls;
+            float m = -INFINITY;
+            for (int q = start + wl; q < Lr; q += 64) m = fmaxf(m, sc[q]);
+            m = wave_max(m);
+            double part = 0.0;
+            for (int q = start + wl; q < Lr; q += 64) {
+                const float e = ref_expf_s(sc[q] - m);
+                sc[q] = e;
+                part += static_cast<double>(e);
+            }
+            const float scale = static_cast<float>(1.0 / wave_sum(part));
+            for (int q = start + wl; q < Lr; q += 64) sc[q] *= scale;
+            for (int q = p_begin + wl; q < start; q += 64) sc[q] = 0.0f;
         }
-        const float scale = static_cast<float>(1.0 / wave_sum(part));
-        for (int q = start + wl; q < Lr; q += 64) sc[q] *= scale;
-        for (int q = wl; q < start; q += 64) sc[q] = 0.0f;
+    } else {  // the whole workgroup on each row; the sum by one wave, in the same grouping
+        __shared__ float px_mx[4];
+        __shared__ float px_scale;
+        for (int r = 0; r < rows; ++r) {
+            int start, Lr;
+            span(r, start, Lr);
+            float* sc = px_sc + r * Ls;
+            float m = -INFINITY;
+            for (int q = start + t; q < Lr; q += kThreads) m = fmaxf(m, sc[q]);
+            m = wave_max(m);
+            if (wl == 0) px_mx[wave] = m;
+            __syncthreads();
+            m = fmaxf(fmaxf(px_mx[0], px_mx[1]), fmaxf(px_mx[2], px_mx[3]));
+            for (int q = start + t; q < Lr; q += kThreads) sc[q] = ref_expf_s(sc[q] - m);
+            for (int q = p_begin + t; q < start; q += kThreads) sc[q] = 0.0f;
+            __syncthreads();
+            if (wave == 0) {
+                double part = 0.0;
+                for (int q = start + wl; q < Lr; q += 64) part += static_cast<double>(sc[q]);
+                part = wave_sum(part);
+                if (wl == 0) px_scale = static_cast<float>(1.0 / part);
+            }
+            __syncthreads();
+            const float scale = px_scale;
+            for (int q = start + t; q < Lr; q += kThreads) sc[q] *= scale;
+        }
     }
     __syncthreads();
     // ---- value sums in position order: lane = (dimension pair dp, rows rg, rg + RG, ...)
-    constexpr int DP = HD / 2, RG = kThreads / DP, NR = R / RG;
+    constexpr int DP = HD / 2, RG = kThreads / DP, NR = R > RG ? R / RG : 1;
     const int dp = t % DP, rg = t / DP;
     float acc0[NR], acc1[NR];
     int lr[NR];
@@ -1946,12 +1987,13 @@ __global__ __launch_bounds__(kThreads) void k_pre_attn_rows(PreAttnArgs p, int n
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
         acc0[k] = acc1[k] = 0.0f;
-        const int row = rg + k * RG < rows ? rg + k * RG : rows - 1;  // past the block: a copy, not stored
-        lr[k] = first + row / hpk + 1;
-        wrow[k] = s.sc + row * Ls;
+        const int r = rg + k * RG < rows ? rg + k * RG : rows - 1;  // past the block: a copy, not stored
+        lr[k] = p.pos0 + px_tok[r] + 1;
+        wrow[k] = px_sc + r * Ls;
         lmin = lr[k] < lmin ? lr[k] : lmin;
         lmax = lr[k] > lmax ? lr[k] : lmax;
     }
+    if (rg >= R) lmin = lmax = p_begin;  // fewer rows than row groups: nothing to sum
     const uint32_t* vcol = reinterpret_cast<const uint32_t*>(vbase) + dp;  // value pair (2 dp, 2 dp + 1) of row 0
     // positions every chain takes, in batches of B: the next batch's loads are
     // issued before the current batch's adds (two register sets, ping-pong),
@@ -1981,8 +2023,8 @@ __global__ __launch_bounds__(kThreads) void k_pre_attn_rows(PreAttnArgs p, int n
             acc1[k] = a1;
         }
     };
-    if (nb > 0) load(va, 0);
-    int b = 0;
+    int b = p_begin / B;
+    if (b < nb) load(va, b * B);
     for (; b + 2 <= nb; b += 2) {
         load(vb, (b + 1) * B);
         adds(va, b * B);
@@ -1990,8 +2032,7 @@ __global__ __launch_bounds__(kThreads) void k_pre_attn_rows(PreAttnArgs p, int n
         adds(vb, (b + 1) * B);
     }
     if (b < nb) adds(va, b * B);
-    int q = nb * B;
-    for (; q < lmax; ++q) {
+    for (int q = nb * B; q < lmax; ++q) {
         const uint32_t v = vcol[static_cast<size_t>(q) * DP];
 #pragma unroll
         for (int k = 0; k < NR; ++k)
@@ -2003,29 +2044,29 @@ __global__ __launch_bounds__(kThreads) void k_pre_attn_rows(PreAttnArgs p, int n
     }
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
-        const int row = rg + k * RG;
-        if (row < rows) {
-            const int tt = row / hpk, gq = row - tt * hpk;
-            float* o = p.out + static_cast<size_t>(tb0 + tt) * p.qstride + (kv * hpk + gq) * HD + 2 * dp;
+        const int r = rg + k * RG;
+        if (r < rows) {
+            const int tt = px_tok[r], gq = row0 + r - tt * hpk;
+            float* o = p.out + static_cast<size_t>(tt) * p.qstride + (kv * hpk + gq) * HD + 2 * dp;
             *reinterpret_cast<float2*>(o) = make_float2(acc0[k], acc1[k]);
         }
     }
     // The O projection's activation blocks: token tt's hpk heads of this kv head are values
     // kv * 256 .. kv * 256 + 255 of its row, one whole block, quantised here (as k_pre_quant_blocks
-    // does from the stored rows) instead of by a separate launch.  s.q is free: its last reads
-    // (the scores) are behind the softmax's barriers.
-    if (p.qout.qs != nullptr && hpk * HD == 256) {
+    // does from the stored rows) instead of by a separate launch, when the block's rows are whole
+    // tokens.  px_q is free: its last reads (the scores) are behind the softmax's barriers.
+    if (p.qout.qs != nullptr && hpk * HD == 256 && R % hpk == 0) {
 #pragma unroll
         for (int k = 0; k < NR; ++k) {
-            const int row = rg + k * RG;
-            if (row < rows) *reinterpret_cast<float2*>(s.q + row * HD + 2 * dp) = make_float2(acc0[k], acc1[k]);
+            const int r = rg + k * RG;
+            if (r < rows) *reinterpret_cast<float2*>(px_q + r * HD + 2 * dp) = make_float2(acc0[k], acc1[k]);
         }
         __syncthreads();
-        for (int tt = wave; tt < ntb; tt += kThreads / 64) {
-            const float4 x = *reinterpret_cast<const float4*>(s.q + tt * 256 + 4 * wl);
+        for (int tt = wave; tt < rows / hpk; tt += kThreads / 64) {
+            const float4 x = *reinterpret_cast<const float4*>(px_q + tt * 256 + 4 * wl);
             const float v[4] = {x.x, x.y, x.z, x.w};
-            if (p.q8k) pre_quant_block<true>(v, tb0 + tt, kv, p.qbits, p.qout);
-            else pre_quant_block<false>(v, tb0 + tt, kv, p.qbits, p.qout);
+            if (p.q8k) pre_quant_block<true>(v, tok0 + tt, kv, p.qbits, p.qout);
+            else pre_quant_block<false>(v, tok0 + tt, kv, p.qbits, p.qout);
         }
     }
 }
@@ -2477,6 +2518,33 @@ hipError_t launch_softcap(float* x, size_t n, float cap, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Query rows a workgroup of k_pre_attn_rows: the most (16, 8, 4, 2 or 1) that give every compute unit two
+// workgroups and keep two of them a unit (their scores in LDS).  Fewer rows read the keys and values
+// more often, so a context whose scores no longer fit twice takes them once rather than halve the rows below 4.
+// Measured at 16 / 8 / 4 / 2 / 1 rows: 6 tokens at 300 positions (Llama-3.2-1B shape, 4 layers) 620 / 570 /
+// 546 / 546 / 553 us a call, a 512-token prompt of it 4.01 / 4.08 / 4.31 / 4.58 / 5.29 ms; 3001 tokens
+// (Qwen3-1.7B shape, 4 layers) 19.0 ms with 8 rows throughout, 18.5 with 4, 23.7 with 2, 17.8 by this rule.
+static int attn_rows(int rows, int kv_heads, int L) {
+    const size_t row_bytes = static_cast<size_t>(attn_row_floats(L) + 128) * 4;
+    int R = 16;
+    while (R > 1 && ((rows + R - 1) / R * kv_heads < 2 * kKqCus || R * row_bytes > (R > 4 ? kAttnRowsLds / 2 : kAttnRowsLds))) R /= 2;
+    return R;
+}
+
+template <int HD>
+static void attn_rows_launch(const PreAttnArgs& p, int ntok, int R, int L, hipStream_t s) {
+    const int rows = ntok * (p.a.heads / p.a.kv_heads), Ls = attn_row_floats(L);
+    const dim3 grid((rows + R - 1) / R * p.a.kv_heads);
+    const size_t lds = static_cast<size_t>(R) * (Ls + HD) * 4;
+    switch (R) {
+        case 16: hipLaunchKernelGGL((k_pre_attn_rows<HD, 16>), grid, dim3(kThreads), lds, s, p, ntok, Ls); break;
+        case 8: hipLaunchKernelGGL((k_pre_attn_rows<HD, 8>), grid, dim3(kThreads), lds, s, p, ntok, Ls); break;
+        case 4: hipLaunchKernelGGL((k_pre_attn_rows<HD, 4>), grid, dim3(kThreads), lds, s, p, ntok, Ls); break;
+        case 2: hipLaunchKernelGGL((k_pre_attn_rows<HD, 2>), grid, dim3(kThreads), lds, s, p, ntok, Ls); break;
+        default: hipLaunchKernelGGL((k_pre_attn_rows<HD, 1>), grid, dim3(kThreads), lds, s, p, ntok, Ls); break;
+    }
+}
+
 hipError_t launch_pre_attention(const PreAttnArgs& p, int ntok, hipStream_t s, bool* quantised) {
     if (quantised != nullptr) *quantised = false;
     if (ntok <= 0) return hipSuccess;
@@ -2492,11 +2560,11 @@ hipError_t launch_pre_attention(const PreAttnArgs& p, int ntok, hipStream_t s, b
         const dim3 fgrid(((ntok + kFaRows / hpk - 1) / (kFaRows / hpk)) * p.a.kv_heads);
         if (hd == 64) hipLaunchKernelGGL(k_pre_attn_fa<64>, fgrid, dim3(kThreads), 0, s, p, ntok);
         else hipLaunchKernelGGL(k_pre_attn_fa<128>, fgrid, dim3(kThreads), 0, s, p, ntok);
-    } else if (!p.legacy && (hd == 64 || hd == 128) && hpk <= kPxRows && kPxRows % hpk == 0 && L <= kPaMaxL) {
-        const dim3 xgrid(((ntok + kPxRows / hpk - 1) / (kPxRows / hpk)) * p.a.kv_heads);
-        if (hd == 64) hipLaunchKernelGGL((k_pre_attn_rows<64, kPxRows, kPaMaxL>), xgrid, dim3(kThreads), 0, s, p, ntok);
-        else hipLaunchKernelGGL((k_pre_attn_rows<128, kPxRows, kPaMaxL>), xgrid, dim3(kThreads), 0, s, p, ntok);
-        if (quantised != nullptr) *quantised = p.qout.qs != nullptr && hpk * hd == 256;
+    } else if (!p.legacy && pre_attn_rows_fits(hd, L)) {
+        const int R = attn_rows(ntok * hpk, p.a.kv_heads, L);
+        if (hd == 64) attn_rows_launch<64>(p, ntok, R, L, s);
+        else attn_rows_launch<128>(p, ntok, R, L, s);
+        if (quantised != nullptr) *quantised = p.qout.qs != nullptr && hpk * hd == 256 && R % hpk == 0;
     } else if (p.a.window == 0 && hpk <= kPaRows && (p.a.head_dim == 32 || p.a.head_dim == 64 || p.a.head_dim == 128) &&
         p.pos0 + ntok <= kPaMaxL) {
         const int tpb = kPaRows / hpk;

@@ -1223,8 +1223,11 @@ void Session::stage(const int32_t* tokens, size_t n, size_t device_pos) {
 // Prompts of two or more tokens whose attention stays on the exact path go
 // through the batched prefill (BRISK_HIP_PREFILL=0 turns it off).
 bool Session::use_prefill(size_t n) const {
-    // the exact-order prefill attention keeps every score of a token's query heads in LDS
-    const bool exact_fits = (position_ + n) * (cfg_.heads / cfg_.kv_heads) <= static_cast<size_t>(kExactScores);
+    // the exact-order prefill attentions keep scores in LDS: a few rows' (64- and 128-wide heads), or
+    // every score of a token's query heads
+    const bool exact_fits = (position_ + n) * (cfg_.heads / cfg_.kv_heads) <= static_cast<size_t>(kExactScores) ||
+                            (!prefill_legacy_ && position_ + n <= (size_t{1} << 30) &&
+                             pre_attn_rows_fits(static_cast<int>(cfg_.head_dim), static_cast<int>(position_ + n)));
     const bool mfma_fits = prefill_mfma_ && pre_attn_mfma_fits(static_cast<int>(cfg_.heads / cfg_.kv_heads), static_cast<int>(cfg_.head_dim));
     // Gemma 3 (sliding layers, post-norms, GELU, soft-capped logits) and LFM2 (short convolutions)
     // take the exact attention only

@@ -1,7 +1,7 @@
 """Long prompts through the batched prefill, against the oracle.
 
-Default path: the exact-order attention kernels (k_pre_attn_blk up to 512
-positions, k_pre_attn beyond), so logits are bit-identical to the oracle's at
+Default path: the exact-order attention kernels (k_pre_attn_rows for 64- and
+128-wide heads, k_pre_attn for others), so logits are bit-identical to the oracle's at
 every prompt length, also for a prompt that continues an existing context.  Gemma 3
 runs here too: its sliding layers see the last `sliding_window` positions
 (src/model.cpp:1084-1088), its projections pass their post-norms, its gate is GELU.
@@ -135,3 +135,23 @@ def test_prefill_gemm_variants_exact(name, env):
             else:
                 os.environ[k] = v
     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("name,first,second", [("tiny-qwen3-long", 2500, 0), ("tiny-qwen3-long", 1300, 3), ("tiny-qwen3-long", 600, 70),
+                                               ("tiny-bitnet", 900, 5), ("tiny-bitnet", 3, 2), ("tiny-qwen2", 1, 17),
+                                               ("tiny-gemma3", 400, 33)])
+def test_prompt_attention_row_blocks(name, first, second):
+    """k_pre_attn_rows at each number of query rows a workgroup it is launched with: contexts whose
+    scores fit 16, 8 and 4 rows of LDS, batches of a few tokens (2 rows and 1), blocks that end inside
+    a token's heads, both head sizes, sliding windows."""
+    f, cfg, table = model.load(synth.model_path(name))
+    ctx = first + second + 8
+    print(f"[prefill] {name}: {first} + {second} prompt ids", flush=True)
+    prompt = synth.prompt_ids(first + second, cfg.vocab, seed=13)
+    o = pyoracle.Oracle(cfg, table, ctx)
+    want = [o.eval(prompt[:first])] + ([o.eval(prompt[first:])] if second else [])
+    o.close()
+    with HipSession((f, cfg, table), max_context=ctx) as s:
+        got = [s.eval(prompt[:first])] + ([s.eval(prompt[first:])] if second else [])
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g.view(np.uint32), w.view(np.uint32))
