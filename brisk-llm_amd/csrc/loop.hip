@@ -1867,6 +1867,28 @@ __device__ __forceinline__ bool wait_pick(const LoopArgs& g, int step, int& toke
     return true;
 }
 
+// The end of a step without an output projection (a prompt token), by one thread: every
+// row of h after the last layer needs every attention output of that layer, so once one
+// of them is written all of the step's cache rows are in memory.  Without this wait a
+// workgroup with no O, gate/up or down tile could stage the last layer's cached rows of
+// the next step before this step's row is among them: the next token is known, so nothing
+// else ties its first layer to this step's last.  The word may already carry a later tag
+// of this launch.
+__device__ __forceinline__ bool wait_step(const LoopArgs& g, int step) {
+    const unsigned want = tag_of(g, step, g.n_layers - 1, 5);
+    unsigned spins = 0;
+    while (true) {
+        const unsigned tag = static_cast<unsigned>(tload(g.ht) >> 32);
+        if ((tag >> 24) == (want >> 24) && tag >= want) return true;
+        if (++spins > kSpinLimit) {
+            atomicExch(g.error, 1);
+            return false;
+        }
+        if ((spins & 63) == 0 && loop_failed(g)) return false;
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+
 // The launch's arguments (the kernel's only argument, at the start of the kernel
 // argument segment), re-addressed through an opaque copy of the segment pointer
 // at each use: the compiler then reads the fields it needs with scalar loads
@@ -1894,6 +1916,7 @@ __global__ __launch_bounds__(kThreads) void k_loop(LoopArgs g_arg) {
             int token = lg().seq[pos];
             bool ok = true;
             if (step > 0 && pos >= lg().fixed) ok = wait_pick(lg(), step - 1, token);
+            else if (step > 0 && step <= lg().first_full) ok = wait_step(lg(), step - 1);
             if (ok && blockIdx.x == 0) {
                 if (step > 0 && pos >= lg().fixed) lg().seq[pos] = token;
                 // re-arm the key this step's phase H uses: its last readers (the
