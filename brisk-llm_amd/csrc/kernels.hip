@@ -578,53 +578,6 @@ __global__ __launch_bounds__(kThreads) void k_ssm(SsmArgs g) {
     }
 }
 
-// Prefill, state sizes 64 and 128: the ntok tokens at positions pos0 .. in order, the state row in
-// registers throughout.  Token t's rows are qkv[t * qkv_dim ..], z[t * heads * DIM ..], alpha
-// ab[t * ab_stride + h] and beta ab[t * ab_stride + heads + h]; outputs out[t * heads * DIM ..].
-// The half of the last token's parity keeps the state before it (the reference's snapshot,
-// src/model.cpp:798-812), the other half the state after it.
-template <int DIM>
-__global__ __launch_bounds__(kThreads) void k_pre_ssm(SsmArgs g, int pos0, int ntok, int ab_stride) {
-    __shared__ SsmLds s;
-    const int h = blockIdx.x, inner = g.heads * DIM, j = threadIdx.x, taps = g.taps;
-    float row[DIM];
-    ssm_row_load<DIM>(g, h, pos0 & 1, pos0 == 0, row);
-    SsmConv cv;
-    ssm_conv_load<DIM>(g, h, pos0, cv);
-    const SsmConst kc = ssm_const<DIM>(g, h);
-    // token t's rows, z and gates, loaded while token t - 1 steps (the step's barriers leave them in flight)
-    struct In {
-        float cur[3], z, a, b;
-    };
-    auto load_in = [&](int t, In& in) {
-        ssm_cur<DIM>(g, h, g.qkv + static_cast<size_t>(t) * g.qkv_dim, in.cur);
-        in.z = g.z[static_cast<size_t>(t) * inner + h * DIM + (j < DIM ? j : 0)];
-        const float* ab = g.ab + static_cast<size_t>(t) * ab_stride;
-        in.a = ab[h];
-        in.b = ab[g.heads + h];
-    };
-    In in;
-    load_in(0, in);
-    for (int t = 0; t < ntok; ++t) {
-        const int pos = pos0 + t;
-        if (t + 1 == ntok) ssm_row_store<DIM>(g, h, pos & 1, row);
-        In next = in;
-        if (t + 1 < ntok) load_in(t + 1, next);
-        const float out = ssm_step<DIM>(g, s, h, in.cur, cv, in.z, in.a, in.b, row, kc);
-        if (j < DIM) g.out[static_cast<size_t>(t) * inner + h * DIM + j] = out;
-        in = next;
-    }
-    ssm_row_store<DIM>(g, h, (pos0 + ntok) & 1, row);
-    // the ring: the batch's last taps positions' rows (older slots keep theirs)
-    if (j < DIM)
-        for (int t = ntok - taps > 0 ? ntok - taps : 0; t < ntok; ++t)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const int ch = c * inner + h * DIM + j;
-                g.ring[static_cast<size_t>((pos0 + t) % taps) * g.qkv_dim + ch] = g.qkv[static_cast<size_t>(t) * g.qkv_dim + ch];
-            }
-}
-
 // Decode, any state size up to 256: the state read twice from memory.
 __global__ __launch_bounds__(kThreads) void k_ssm_any(SsmArgs g) {
     __shared__ float qs[kThreads], ks[kThreads];
@@ -1256,15 +1209,6 @@ hipError_t launch_ssm(const SsmArgs& g, hipStream_t s) {
     if (g.dim == 64) hipLaunchKernelGGL(k_ssm<64>, grid, block, 0, s, g);
     else if (g.dim == 128) hipLaunchKernelGGL(k_ssm<128>, grid, block, 0, s, g);
     else hipLaunchKernelGGL(k_ssm_any, grid, block, 0, s, g);
-    return hipGetLastError();
-}
-
-hipError_t launch_pre_ssm(const SsmArgs& g, int pos0, int ntok, int ab_stride, hipStream_t s) {
-    if (!pre_ssm_fits(g.dim) || g.heads < 1 || g.taps < 2 || g.taps > 8 || g.qkv_dim != 3 * g.heads * g.dim || ntok < 1 || pos0 < 0)
-        return hipErrorInvalidValue;
-    const dim3 grid(static_cast<unsigned>(g.heads)), block(kThreads);
-    if (g.dim == 64) hipLaunchKernelGGL(k_pre_ssm<64>, grid, block, 0, s, g, pos0, ntok, ab_stride);
-    else hipLaunchKernelGGL(k_pre_ssm<128>, grid, block, 0, s, g, pos0, ntok, ab_stride);
     return hipGetLastError();
 }
 

@@ -160,11 +160,6 @@ hipError_t launch_conv(const float* bcx, uint16_t* cache, const float* w, int ta
                        hipStream_t s);
 // Qwen3.5: one recurrent layer's conv, delta-rule state update and gated norm (one workgroup a head).
 hipError_t launch_ssm(const SsmArgs& g, hipStream_t s);
-// Qwen3.5 prefill: the recurrence over ntok tokens at positions pos0 .. in one launch (state sizes
-// 64 and 128): g.qkv [ntok][qkv_dim], g.z [ntok][heads * dim], alpha and beta of token t at
-// g.ab[t * ab_stride + h] and g.ab[t * ab_stride + heads + h], out [ntok][heads * dim].
-hipError_t launch_pre_ssm(const SsmArgs& g, int pos0, int ntok, int ab_stride, hipStream_t s);
-inline bool pre_ssm_fits(int dim) { return dim == 64 || dim == 128; }
 // Qwen3.5 attention: [heads][q | gate] rows split into q and gate; att *= sigmoid(gate).
 hipError_t launch_qgate_split(const float* qg, float* q, float* gate, int heads, int hd, hipStream_t s);
 hipError_t launch_sigmoid_gate(float* att, const float* gate, int n, hipStream_t s);

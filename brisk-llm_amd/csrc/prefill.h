@@ -114,6 +114,17 @@ hipError_t launch_pre_conv(const float* bcx, uint16_t* cache, const float* w, in
                            hipStream_t s);
 // x[i] = cap tanh(x[i] / cap) (Gemma's final logit soft-capping)
 hipError_t launch_softcap(float* x, size_t n, float cap, hipStream_t s);
+// Qwen3.5 prefill: the recurrence over the ntok tokens at positions pos0 .. (state sizes 64 and 128).
+// s.qkv [ntok][qkv_dim], s.z [ntok][heads * dim], alpha and beta of token t at s.ab[t * ab_stride + h] and
+// s.ab[t * ab_stride + heads + h], s.out [ntok][heads * dim]; conv and gates are scratch.
+struct PreSsmArgs {
+    SsmArgs s;
+    int pos0, ntok, ab_stride;
+    float* conv;   // [ntok][3 * heads * dim]
+    float* gates;  // [ntok][2 * heads]
+};
+inline bool pre_ssm_fits(int dim) { return dim == 64 || dim == 128; }
+hipError_t launch_pre_ssm(const PreSsmArgs& p, hipStream_t s);
 hipError_t launch_pre_attention(const PreAttnArgs& p, int ntok, hipStream_t s, bool* quantised = nullptr);
 
 }  // namespace bh

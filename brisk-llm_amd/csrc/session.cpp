@@ -200,7 +200,7 @@ brisk_hip_memory estimate_session(const brisk_hip_config& cfg, const brisk_hip_t
     if (cfg.arch == BRISK_HIP_ARCH_GEMMA4)  // prefill per-layer embedding inputs and gate rows
         sc += T * static_cast<size_t>(cfg.ple_dim) * (cfg.layers + 1) * 4;
     if (cfg.arch == BRISK_HIP_ARCH_QWEN35)  // prefill recurrence rows, query|gate rows, the wider attention output
-        sc += T * (5 * static_cast<size_t>(cfg.ssm_inner) + 2 * cfg.ssm_v_heads + 2 * qd) * 4;
+        sc += T * (8 * static_cast<size_t>(cfg.ssm_inner) + 4 * cfg.ssm_v_heads + 2 * qd) * 4;
     if (ff > static_cast<size_t>(kMaxCols)) sc += (ff + 255) / 256 * 256 * (1 + 4 / 32.0 + 4 / 16.0);  // wide down input
     sc += static_cast<size_t>(64) * cfg.vocab * 4;                         // eval_all logits
     for (size_t i = 0; i < n; ++i)  // the prefill's expanded layer matrices
@@ -1263,6 +1263,8 @@ void Session::ensure_prefill() {
         pre_sqkv_ = static_cast<float*>(alloc(T * 3 * inner * 4));
         pre_sz_ = static_cast<float*>(alloc(T * inner * 4));
         pre_sab_ = static_cast<float*>(alloc(T * 2 * heads * 4));
+        pre_sconv_ = static_cast<float*>(alloc(T * 3 * inner * 4));
+        pre_sgate_ = static_cast<float*>(alloc(T * 2 * heads * 4));
         pre_qg_ = static_cast<float*>(alloc(T * 2 * qd * 4));
     }
     const size_t widest = std::max(std::max(std::max(e, qd), ff), static_cast<size_t>(cfg_.ssm_inner));
@@ -1324,12 +1326,14 @@ void Session::prefill_layers(size_t pos0, int T) {
                 g.m = m.p; set_mx(g, m); g.out = outs[i]; g.ostride = strides[i];
                 check(launch_mm(g, kMmStore, stream_), "prefill recurrence projections");
             }
-            SsmArgs sa{};
+            PreSsmArgs ps{};
+            SsmArgs& sa = ps.s;
             sa.qkv = pre_sqkv_; sa.z = pre_sz_; sa.ab = pre_sab_; sa.conv_w = L.ssm_conv_w; sa.a = L.ssm_a; sa.dt = L.ssm_dt;
             sa.norm = L.ssm_norm; sa.ring = L.ssm_ring; sa.state = L.ssm_state; sa.pos = pos_; sa.out = pre_att_;
             sa.heads = heads; sa.dim = static_cast<int>(cfg_.ssm_state); sa.taps = static_cast<int>(cfg_.ssm_conv); sa.qkv_dim = qkv;
             sa.eps = cfg_.rms_epsilon; sa.q_scale = 1.0f / std::sqrt(static_cast<float>(cfg_.ssm_state));  // src/model.cpp:813
-            check(launch_pre_ssm(sa, static_cast<int>(pos0), T, 2 * heads, stream_), "prefill recurrence");
+            ps.pos0 = static_cast<int>(pos0); ps.ntok = T; ps.ab_stride = 2 * heads; ps.conv = pre_sconv_; ps.gates = pre_sgate_;
+            check(launch_pre_ssm(ps, stream_), "prefill recurrence");
             prefill_quant(pre_att_, inner, nullptr, inner, T, L.ssm_out);
             g.m = L.ssm_out.p; set_mx(g, L.ssm_out); g.out = pre_h_; g.ostride = e;
             check(launch_mm(g, kMmAdd, stream_), "prefill ssm_out");

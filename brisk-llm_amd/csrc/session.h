@@ -189,7 +189,7 @@ private:
     float* pre_proj_ = nullptr;  // Gemma: a projection's rows before their post-norm; LFM2: conv outputs
     float* pre_conv_ = nullptr;  // LFM2: in_proj rows [b | c | x]
     // Qwen3.5: the recurrence's projections [T][qkv], [T][inner], [T][alpha | beta]; the query|gate rows
-    float *pre_sqkv_ = nullptr, *pre_sz_ = nullptr, *pre_sab_ = nullptr, *pre_qg_ = nullptr;
+    float *pre_sqkv_ = nullptr, *pre_sz_ = nullptr, *pre_sab_ = nullptr, *pre_qg_ = nullptr, *pre_sconv_ = nullptr, *pre_sgate_ = nullptr;
     float *pre_ple_ = nullptr, *pre_pleg_ = nullptr;  // Gemma 4: per-layer embedding inputs and gate rows
     ActPlanar pre_x_{};
     ActPlanar wide_x_{};  // feed-forward rows past kMaxCols: the down projection's quantised input (one token)
