@@ -182,179 +182,89 @@ __global__ void k_pre_planar(const uint8_t* __restrict__ xq, int cols, int q8k, 
 
 // ---------------------------------------------------------------- weight fragments
 
-// Eight consecutive weight values (k = kq .. kq + 7 of 32-value sub-block j) of
-// one row as signed int8, the A operand of one lane.  Q4_0: nibble - 8;
-// Q4_1: nibble 0..15 (the offset m enters through the block sum); Q5_0: 5-bit
-// value - 16; Q8_0: as stored; Q4_K: nibble 0..15, Q5_K: 5-bit value 0..31
-// (the mins enter through the offsets);
-// Q6_K: 6-bit value - 32; TQ2_0: code - 1.  Sign extension is done per byte
-// (SWAR): for a field t of n bits, t | ((t & sign) * k) with k filling the
-// high bits.
 constexpr uint64_t kB01 = 0x0101010101010101ull;
 
 __device__ __forceinline__ uint64_t ld8(const uint8_t* p) { return *reinterpret_cast<const uint64_t*>(p); }
 
-template <uint32_t T>
-__device__ __forceinline__ uint64_t frag_a(const Packed& m, uint32_t row, uint32_t j, int kq) {
-    if (T == kQ8_0) {
-        const uint32_t nsub = m.cols / 32;
-        return ld8(m.p0 + (static_cast<size_t>(row) * nsub + j) * 32 + kq);
-    } else if (T == kQ4_0) {
-        const uint32_t nsub = m.cols / 32;
-        const uint64_t w = ld8(m.p0 + (static_cast<size_t>(row) * nsub + j) * 16 + (kq & 15));
-        const uint64_t nib = kq < 16 ? (w & (0x0F * kB01)) : ((w >> 4) & (0x0F * kB01));
-        const uint64_t t = nib ^ (0x08 * kB01);             // 4-bit two's complement of nib - 8
-        return t | ((t & (0x08 * kB01)) * 0x1E);             // sign-extend bit 3
-    } else if (T == kQ4_1) {
-        const uint32_t nsub = m.cols / 32;
-        const uint64_t w = ld8(m.p0 + (static_cast<size_t>(row) * nsub + j) * 16 + (kq & 15));
-        return kq < 16 ? (w & (0x0F * kB01)) : ((w >> 4) & (0x0F * kB01));
-    } else if (T == kQ5_0) {
-        const uint32_t nsub = m.cols / 32;
-        const size_t blk = static_cast<size_t>(row) * nsub + j;
-        const uint64_t w = ld8(m.p0 + blk * 16 + (kq & 15));
-        const uint32_t qh = reinterpret_cast<const uint32_t*>(m.p2)[blk] >> kq;  // bits of values kq .. kq + 7
-        const uint64_t hb = static_cast<uint64_t>(spread4_hi(qh, 0)) | (static_cast<uint64_t>(spread4_hi(qh, 4)) << 32);
-        const uint64_t u = (kq < 16 ? (w & (0x0F * kB01)) : ((w >> 4) & (0x0F * kB01))) | hb;  // 0..31
-        const uint64_t t = u ^ (0x10 * kB01);                                                // 5-bit two's complement of u - 16
-        return t | ((t & (0x10 * kB01)) * 0x0E);
-    } else if (T == kQ4_K) {
-        const uint32_t nsb = m.cols / 256, jj = j & 7;
-        const size_t blk = static_cast<size_t>(row) * nsb + j / 8;
-        const uint64_t w = ld8(m.p0 + blk * 128 + (jj >> 1) * 32 + kq);
-        return (jj & 1) ? ((w >> 4) & (0x0F * kB01)) : (w & (0x0F * kB01));
-    } else if (T == kQ5_K) {
-        const uint32_t nsb = m.cols / 256, jj = j & 7;
-        const size_t blk = static_cast<size_t>(row) * nsb + j / 8;
-        const uint64_t w = ld8(m.p0 + blk * 128 + (jj >> 1) * 32 + kq);
-        const uint64_t h = ld8(m.p2 + blk * 48 + 16 + kq);
-        const uint64_t nib = (jj & 1) ? ((w >> 4) & (0x0F * kB01)) : (w & (0x0F * kB01));
-        return nib | (((h >> jj) & kB01) << 4);
-    } else if (T == kQ6_K) {
-        const uint32_t nsb = m.cols / 256, jj = j & 7, half = jj >> 2, quarter = jj & 3;
-        const size_t blk = static_cast<size_t>(row) * nsb + j / 8;
-        const uint64_t l = ld8(m.p0 + blk * 128 + half * 64 + (quarter & 1) * 32 + kq);
-        const uint64_t h = ld8(m.p1 + blk * 64 + half * 32 + kq);
-        const uint64_t nib = quarter >= 2 ? ((l >> 4) & (0x0F * kB01)) : (l & (0x0F * kB01));
-        const uint64_t u = nib | (((h >> (2 * quarter)) & (0x03 * kB01)) << 4);  // 0..63
-        const uint64_t t = u ^ (0x20 * kB01);                                   // 6-bit two's complement of u - 32
-        return t | ((t & (0x20 * kB01)) * 0x06);
-    } else {  // TQ2_0
-        const uint32_t nsb = m.cols / 256, jj = j & 7;
-        const size_t blk = static_cast<size_t>(row) * nsb + j / 8;
-        const uint64_t w = ld8(m.p0 + blk * 64 + (jj >> 2) * 32 + kq);
-        const uint64_t c = (w >> (2 * (jj & 3))) & (0x03 * kB01);                // 0..2
-        const uint64_t t = (c + 0x03 * kB01) & (0x03 * kB01);                   // 2-bit two's complement of c - 1
-        return t | ((t & (0x02 * kB01)) * 0x7F);
-    }
+// Eight consecutive values (k = kq .. kq + 7 of 32-value sub-block j) of one Q5_K row as int8 0..31, the
+// A operand of one lane (the mins enter through the offsets).
+__device__ __forceinline__ uint64_t q5k_frag(const Packed& m, uint32_t row, uint32_t j, int kq) {
+    const uint32_t nsb = m.cols / 256, jj = j & 7;
+    const size_t blk = static_cast<size_t>(row) * nsb + j / 8;
+    const uint64_t w = ld8(m.p0 + blk * 128 + (jj >> 1) * 32 + kq);
+    const uint64_t h = ld8(m.p2 + blk * 48 + 16 + kq);
+    const uint64_t nib = (jj & 1) ? ((w >> 4) & (0x0F * kB01)) : (w & (0x0F * kB01));
+    return nib | (((h >> jj) & kB01) << 4);
 }
 
 __device__ __forceinline__ v4i mfma(uint64_t a, uint64_t b, v4i c) {
     return __builtin_amdgcn_mfma_i32_16x16x32_i8(static_cast<long>(a), static_cast<long>(b), c, 0, 0, 0);
 }
 
-// ---------------------------------------------------------------- the GEMM
+// ---------------------------------------------------------------- the GEMM of unexpanded Q5_K
 
-// A workgroup computes 64 rows (4 waves x 16) x 64 tokens (4 groups of 16).
-// The K dimension goes in chunks of 256 values (8 sub-blocks; one super-block
-// for the K-quants).  Per chunk the workgroup stages the 64 tokens'
-// activations (and their scales) in LDS, and each lane holds its weight
-// fragments and row scales in registers; both are loaded one chunk ahead, so
-// memory latency overlaps the MFMAs and the float epilogue.
+// A workgroup computes 64 rows (4 waves x 16) x 32 tokens (2 groups of 16).
+// The K dimension goes in chunks of 256 values (a super-block).  Per chunk the
+// workgroup stages the tokens' activations (and their scales) in LDS, and each
+// lane holds its weight fragments and row scales in registers; both are loaded
+// one chunk ahead, so memory latency overlaps the MFMAs and the float epilogue.
 constexpr int kRowsPerWg = 64;
 constexpr int kChunkCols = kMmChunkCols;
 constexpr int kBRow = kChunkCols + 16;  // LDS bytes per token row, padded off the bank period
-// Token groups of 16 a workgroup: 4 (64 tokens), or 2 for the K-quants, whose
-// integer epilogue holds more state per output.
-template <uint32_t T>
-__host__ __device__ constexpr int mm_groups() { return (T == kQ4_K || T == kQ5_K || T == kQ6_K) ? 2 : 4; }
+constexpr int kQ5Groups = 2;  // token groups of 16 a workgroup (the integer epilogue's state is per output)
+constexpr int kQ5Tok = 16 * kQ5Groups;
 
-template <int G>
-struct MmLds {
-    alignas(16) int8_t b[16 * G][kBRow];
-    float xd[16 * G][8];     // Q8_0: the chunk's 8 block scales; Q8_K: [0] the super-block's
-    int32_t bs[16 * G][16];  // Q8_K: the super-block's bsums; Q8_0 (for Q4_1): [0..7] the 8 block sums
+struct Q5Lds {
+    alignas(16) int8_t b[kQ5Tok][kBRow];
+    float xd[kQ5Tok];
+    int32_t bs[kQ5Tok][16];  // the super-block's bsums
 };
 
 // One thread's share of a chunk's activations, in flight to LDS.
-template <int G>
 struct ActStage {
-    uint4 q[G];
-    float d[2];
-    int32_t bs[4];  // Q8_0 with sums: [0..1] as d
+    uint4 q[kQ5Groups];
+    float d;
+    int32_t bs[4];
 };
 
-template <int G>
-__device__ __forceinline__ void act_stage_load(ActStage<G>& st, const ActPlanar& x, int ntok, int t0, int c, bool q8k,
-                                               bool sums = false) {
-    constexpr int kTok = 16 * G;
+__device__ __forceinline__ void act_stage_load(ActStage& st, const ActPlanar& x, int ntok, int t0, int c) {
     const int tid = threadIdx.x;
 #pragma unroll
-    for (int k = 0; k < G; ++k) {
+    for (int k = 0; k < kQ5Groups; ++k) {
         const int idx = k * kThreads + tid, tok = idx >> 4, piece = idx & 15;
         const int t = t0 + tok < ntok ? t0 + tok : ntok - 1;
         st.q[k] = *reinterpret_cast<const uint4*>(x.qs + static_cast<size_t>(t) * x.stride + c * kChunkCols + piece * 16);
     }
     const size_t ds = x.stride / 32, bss = x.stride / 16;
-    if (!q8k) {  // kTok tokens x 8 scales
+    const int tok = tid >> 2;
+    if (tok < kQ5Tok) {
+        const int t = t0 + tok < ntok ? t0 + tok : ntok - 1;
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int idx = k * kThreads + tid, tok = idx >> 3, blk = idx & 7;
-            if (tok < kTok) {
-                const int t = t0 + tok < ntok ? t0 + tok : ntok - 1;
-                st.d[k] = x.d[t * ds + c * 8 + blk];
-                if (sums) st.bs[k] = x.bs[t * bss + c * 8 + blk];
-            }
-        }
-    } else {  // kTok tokens x 16 bsums, and kTok scales
-        const int tok = tid >> 2;
-        if (tok < kTok) {
-            const int t = t0 + tok < ntok ? t0 + tok : ntok - 1;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) st.bs[k] = x.bs[t * bss + c * 16 + (tid & 3) * 4 + k];
-        }
-        if (tid < kTok) {
-            const int t2 = t0 + tid < ntok ? t0 + tid : ntok - 1;
-            st.d[0] = x.d[t2 * ds + c];
-        }
+        for (int k = 0; k < 4; ++k) st.bs[k] = x.bs[t * bss + c * 16 + (tid & 3) * 4 + k];
     }
+    if (tid < kQ5Tok) st.d = x.d[(t0 + tid < ntok ? t0 + tid : ntok - 1) * ds + c];
 }
 
-template <int G>
-__device__ __forceinline__ void act_stage_store(const ActStage<G>& st, MmLds<G>& L, bool q8k, bool sums = false) {
-    constexpr int kTok = 16 * G;
+__device__ __forceinline__ void act_stage_store(const ActStage& st, Q5Lds& L) {
     const int tid = threadIdx.x;
 #pragma unroll
-    for (int k = 0; k < G; ++k) {
+    for (int k = 0; k < kQ5Groups; ++k) {
         const int idx = k * kThreads + tid, tok = idx >> 4, piece = idx & 15;
         *reinterpret_cast<uint4*>(&L.b[tok][piece * 16]) = st.q[k];
     }
-    if (!q8k) {
+    if ((tid >> 2) < kQ5Tok) {
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int idx = k * kThreads + tid;
-            if ((idx >> 3) < kTok) {
-                L.xd[idx >> 3][idx & 7] = st.d[k];
-                if (sums) L.bs[idx >> 3][idx & 7] = st.bs[k];
-            }
-        }
-    } else {
-        if ((tid >> 2) < kTok) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) L.bs[tid >> 2][(tid & 3) * 4 + k] = st.bs[k];
-        }
-        if (tid < kTok) L.xd[tid][0] = st.d[0];
+        for (int k = 0; k < 4; ++k) L.bs[tid >> 2][(tid & 3) * 4 + k] = st.bs[k];
     }
+    if (tid < kQ5Tok) L.xd[tid] = st.d;
 }
 
 // One lane's weights for a chunk: the A fragments of its row (8 sub-blocks) and
 // the scales of its 4 output rows.
-template <uint32_t T>
 struct WChunk {
     uint64_t a[8];
-    uint4 sc[4];     // Q4_0/Q4_1/Q5_0/Q8_0: 8 fp16 block scales a row; Q4_K/Q5_K: the decoded scales and mins; TQ2_0: .x = d
-    uint32_t s6[4];  // Q6_K: the fp16 d of each row (its int8 scales go in sc); Q4_K/Q5_K: {d, dmin}
-    uint4 mn[4];     // Q4_1: 8 fp16 block offsets m a row
+    uint4 sc[4];     // the decoded scales and mins
+    uint32_t s6[4];  // {d, dmin}
 };
 
 // The 8 fp16 values of a row's plane at element e0 (a chunk's block scales), or its first nb of
@@ -367,42 +277,16 @@ __device__ __forceinline__ uint4 chunk_halves(const uint8_t* plane, size_t e0, i
     return make_uint4(wd[0], wd[1], wd[2], wd[3]);
 }
 
-// Chunk c's weights; nb of its 8 sub-blocks lie in the row (fewer than 8 only in the last chunk
-// of a row of 32-value blocks that is not whole 256-value chunks): the others are not read.
-template <uint32_t T>
-__device__ __forceinline__ void wchunk_load(WChunk<T>& w, const Packed& m, uint32_t arow, bool arow_ok, const uint32_t orow[4],
-                                            int c, int kq, int nb = 8) {
+__device__ __forceinline__ void wchunk_load(WChunk& w, const Packed& m, uint32_t arow, bool arow_ok, const uint32_t orow[4],
+                                            int c, int kq) {
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj) w.a[jj] = arow_ok && jj < nb ? frag_a<T>(m, arow, c * 8 + jj, kq) : 0ull;
-    if (T == kQ4_0 || T == kQ4_1 || T == kQ5_0 || T == kQ8_0) {
-        const uint32_t nsub = m.cols / 32;
+    for (int jj = 0; jj < 8; ++jj) w.a[jj] = arow_ok ? q5k_frag(m, arow, c * 8 + jj, kq) : 0ull;
+    const uint32_t nsb = m.cols / 256;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w.sc[i] = chunk_halves(m.p1, static_cast<size_t>(orow[i]) * nsub + c * 8, nb);
-        if (T == kQ4_1) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) w.mn[i] = chunk_halves(m.p2, static_cast<size_t>(orow[i]) * nsub + c * 8, nb);
-        }
-    } else if (T == kQ4_K || T == kQ5_K) {
-        const uint32_t nsb = m.cols / 256;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const size_t blk = static_cast<size_t>(orow[i]) * nsb + c;
-            w.sc[i] = *reinterpret_cast<const uint4*>(m.p2 + blk * (T == kQ5_K ? 48 : 16));
-            w.s6[i] = *reinterpret_cast<const uint32_t*>(m.p1 + blk * 16);
-        }
-    } else if (T == kQ6_K) {
-        const uint32_t nsb = m.cols / 256;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t* mp = reinterpret_cast<const uint32_t*>(m.p2 + (static_cast<size_t>(orow[i]) * nsb + c) * 20);
-            w.sc[i] = make_uint4(mp[0], mp[1], mp[2], mp[3]);
-            w.s6[i] = mp[4];
-        }
-    } else {
-        const uint32_t nsb = m.cols / 256;
-        const uint16_t* dw = reinterpret_cast<const uint16_t*>(m.p1);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w.sc[i].x = dw[static_cast<size_t>(orow[i]) * nsb + c];
+    for (int i = 0; i < 4; ++i) {
+        const size_t blk = static_cast<size_t>(orow[i]) * nsb + c;
+        w.sc[i] = *reinterpret_cast<const uint4*>(m.p2 + blk * 48);
+        w.s6[i] = *reinterpret_cast<const uint32_t*>(m.p1 + blk * 16);
     }
 }
 
@@ -416,144 +300,54 @@ struct MmAcc {
 
 // The chunk's contribution to the lane's outputs (tokens 16 g + l % 16, rows 4 (l / 16) + i),
 // in the reference's term and sum order.
-template <uint32_t T, int G>
-__device__ __forceinline__ void wchunk_compute(const WChunk<T>& w, const MmLds<G>& L, MmAcc<G>& acc, bool lut16, int nb = 8) {
-    constexpr int kGroups = G;
+__device__ __forceinline__ void wchunk_compute(const WChunk& w, const Q5Lds& L, MmAcc<kQ5Groups>& acc) {
+    constexpr int kGroups = kQ5Groups;
     const int lane = threadIdx.x & 63, kq = (lane >> 4) * 8, tl = lane & 15;
     const v4i zero = {0, 0, 0, 0};
-    if (T == kQ4_0 || T == kQ5_0 || T == kQ8_0 || T == kQ4_1) {
+    int wsum[kGroups][4], osum[kGroups][4];
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
-            if (jj >= nb) break;  // past the row (a partial last chunk): no term
-            v4i d[kGroups];
+    for (int g = 0; g < kGroups; ++g)
 #pragma unroll
-            for (int g = 0; g < kGroups; ++g)
-                d[g] = mfma(w.a[jj], *reinterpret_cast<const uint64_t*>(&L.b[16 * g + tl][jj * 32 + kq]), zero);
-            float wd[4], wm[4];
+        for (int i = 0; i < 4; ++i) wsum[g][i] = osum[g][i] = 0;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t word = u4_word(w.sc[i], jj >> 1);
-                wd[i] = h2f(static_cast<uint16_t>((jj & 1) ? (word >> 16) : (word & 0xFFFF)));
-                if (T == kQ4_1) {
-                    const uint32_t mword = u4_word(w.mn[i], jj >> 1);
-                    wm[i] = h2f(static_cast<uint16_t>((jj & 1) ? (mword >> 16) : (mword & 0xFFFF)));
-                }
-            }
+    for (int jj = 0; jj < 8; ++jj) {
+        int sc[4], mn[4];
 #pragma unroll
-            for (int g = 0; g < kGroups; ++g) {
-                const float xd = L.xd[16 * g + tl][jj];
-                if (T == kQ4_1) {  // src/quant.cpp:445-456 with the offset term
-                    const float xs = xd * static_cast<float>(L.bs[16 * g + tl][jj]);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc.s[g][i] += static_cast<float>(d[g][i]) * wd[i] * xd + wm[i] * xs;
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc.s[g][i] += static_cast<float>(d[g][i]) * wd[i] * xd;  // src/quant.cpp:445-482
-                }
-            }
-        }
-    } else if (T == kQ4_K || T == kQ5_K) {
-        int wsum[kGroups][4], osum[kGroups][4];
-#pragma unroll
-        for (int g = 0; g < kGroups; ++g)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) wsum[g][i] = osum[g][i] = 0;
-#pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
-            int sc[4], mn[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                sc[i] = static_cast<int>((u4_word(w.sc[i], jj >> 2) >> (8 * (jj & 3))) & 0xFF);
-                mn[i] = static_cast<int>((u4_word(w.sc[i], 2 + (jj >> 2)) >> (8 * (jj & 3))) & 0xFF);
-            }
-#pragma unroll
-            for (int g = 0; g < kGroups; ++g) {
-                const int t = 16 * g + tl;
-                const v4i d = mfma(w.a[jj], *reinterpret_cast<const uint64_t*>(&L.b[t][jj * 32 + kq]), zero);
-                const int pair = L.bs[t][2 * jj] + L.bs[t][2 * jj + 1];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    wsum[g][i] += sc[i] * d[i];
-                    osum[g][i] += mn[i] * pair;
-                }
-            }
+        for (int i = 0; i < 4; ++i) {
+            sc[i] = static_cast<int>((u4_word(w.sc[i], jj >> 2) >> (8 * (jj & 3))) & 0xFF);
+            mn[i] = static_cast<int>((u4_word(w.sc[i], 2 + (jj >> 2)) >> (8 * (jj & 3))) & 0xFF);
         }
 #pragma unroll
         for (int g = 0; g < kGroups; ++g) {
-            const float xd = L.xd[16 * g + tl][0];
+            const int t = 16 * g + tl;
+            const v4i d = mfma(w.a[jj], *reinterpret_cast<const uint64_t*>(&L.b[t][jj * 32 + kq]), zero);
+            const int pair = L.bs[t][2 * jj] + L.bs[t][2 * jj + 1];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float d = h2f(static_cast<uint16_t>(w.s6[i] & 0xFFFF)), dmin = h2f(static_cast<uint16_t>(w.s6[i] >> 16));
-                acc.s[g][i] += xd * (d * static_cast<float>(wsum[g][i]) - dmin * static_cast<float>(osum[g][i]));  // :500-521
+                wsum[g][i] += sc[i] * d[i];
+                osum[g][i] += mn[i] * pair;
             }
         }
-    } else if (T == kQ6_K) {
-        const bool lo_half = lane < 32;  // lanes 0..31 hold k 0..15 of a sub-block, 32..63 hold k 16..31
-        int wsum[kGroups][4];
+    }
 #pragma unroll
-        for (int g = 0; g < kGroups; ++g)
+    for (int g = 0; g < kGroups; ++g) {
+        const float xd = L.xd[16 * g + tl];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) wsum[g][i] = 0;
-#pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
-            const uint64_t a0 = lo_half ? w.a[jj] : 0ull, a1 = lo_half ? 0ull : w.a[jj];  // groups 2 jj and 2 jj + 1 of 16
-            int s0[4], s1[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t word = u4_word(w.sc[i], jj >> 1);
-                const int sh = (jj & 1) * 16;
-                s0[i] = static_cast<int8_t>((word >> sh) & 0xFF);
-                s1[i] = static_cast<int8_t>((word >> (sh + 8)) & 0xFF);
-            }
-#pragma unroll
-            for (int g = 0; g < kGroups; ++g) {
-                const uint64_t b = *reinterpret_cast<const uint64_t*>(&L.b[16 * g + tl][jj * 32 + kq]);
-                const v4i d0 = mfma(a0, b, zero), d1 = mfma(a1, b, zero);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) wsum[g][i] += s0[i] * d0[i] + s1[i] * d1[i];
-            }
-        }
-#pragma unroll
-        for (int g = 0; g < kGroups; ++g) {
-            const float xd = L.xd[16 * g + tl][0];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float d = h2f(static_cast<uint16_t>(w.s6[i] & 0xFFFF));
-                acc.s[g][i] += xd * d * static_cast<float>(wsum[g][i]);  // src/quant.cpp:549-563
-            }
-        }
-    } else {  // TQ2_0
-        v4i d[kGroups];
-#pragma unroll
-        for (int g = 0; g < kGroups; ++g) d[g] = zero;
-#pragma unroll
-        for (int jj = 0; jj < 8; ++jj)  // the block's int32 sum over its 8 sub-blocks, exact
-#pragma unroll
-            for (int g = 0; g < kGroups; ++g)
-                d[g] = mfma(w.a[jj], *reinterpret_cast<const uint64_t*>(&L.b[16 * g + tl][jj * 32 + kq]), d[g]);
-#pragma unroll
-        for (int g = 0; g < kGroups; ++g) {
-            const float xd = L.xd[16 * g + tl][0];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float wv = h2f(static_cast<uint16_t>(w.sc[i].x & 0xFFFF));
-                const float a = static_cast<float>(d[g][i]);
-                acc.s[g][i] += lut16 ? a * wv * xd : xd * wv * a;  // src/quant.cpp:789-802 / :580-596
-            }
+        for (int i = 0; i < 4; ++i) {
+            const float d = h2f(static_cast<uint16_t>(w.s6[i] & 0xFFFF)), dmin = h2f(static_cast<uint16_t>(w.s6[i] >> 16));
+            acc.s[g][i] += xd * (d * static_cast<float>(wsum[g][i]) - dmin * static_cast<float>(osum[g][i]));  // :500-521
         }
     }
 }
 
-// out[t * ostride + r] (=, += or gate(out) * up) for a 64-row x 64-token tile.
-template <uint32_t T, int MODE>
+// out[t * ostride + r] (=, += or gate(out) * up) for a 64-row x 32-token tile.
+template <int MODE>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_mm(MmArgs g) {
-    constexpr int kGroups = mm_groups<T>(), kTokPerWg = 16 * kGroups;
-    __shared__ MmLds<kGroups> L;
+    constexpr int kGroups = kQ5Groups;
+    __shared__ Q5Lds L;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, kq = (lane >> 4) * 8;
     const uint32_t r0 = blockIdx.x * kRowsPerWg + wave * 16;
-    const int t0 = blockIdx.y * kTokPerWg;
-    const bool q8k = takes_q8_k(T);
-    const bool lut16 = (g.m.flags & kFlagLut16) != 0;
+    const int t0 = blockIdx.y * kQ5Tok;
     // rows of this lane: the A fragment's, and the 4 outputs' (clamped for the scale loads; never stored)
     const uint32_t rmax = g.m.rows - 1;
     const bool wave_ok = r0 <= rmax;
@@ -571,45 +365,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 2))
     for (int gi = 0; gi < kGroups; ++gi)
 #pragma unroll
         for (int i = 0; i < 4; ++i) a.s[gi][i] = 0.0f;
-    // chunks of 256 values; a row of 32-value blocks may end inside its last chunk (nb_of < 8
-    // blocks there; its activation reads stay inside the planar rows, whose stride is whole chunks)
-    const int nc = static_cast<int>((g.m.cols + kChunkCols - 1) / kChunkCols), nsub = static_cast<int>(g.m.cols / 32);
-    auto nb_of = [&](int c) { return nsub - 8 * c < 8 ? nsub - 8 * c : 8; };
-    ActStage<kGroups> st;
-    WChunk<T> w0, w1;  // two chunks in flight
-    constexpr bool kSums = T == kQ4_1;
-    act_stage_load(st, g.x, g.ntok, t0, 0, q8k, kSums);
-    if (wave_ok) {
-        wchunk_load<T>(w0, g.m, arow, arow_ok, orow, 0, kq, nb_of(0));
-    }
+    const int nc = static_cast<int>(g.m.cols / kChunkCols);
+    ActStage st;
+    WChunk w0, w1;  // two chunks in flight
+    act_stage_load(st, g.x, g.ntok, t0, 0);
+    if (wave_ok) wchunk_load(w0, g.m, arow, arow_ok, orow, 0, kq);
     for (int c = 0; c < nc; c += 2) {
-        // chunk c (weights in w0/v0)
+        // chunk c (weights in w0)
         __syncthreads();
-        act_stage_store(st, L, q8k, kSums);
+        act_stage_store(st, L);
         __syncthreads();
         if (c + 1 < nc) {
-            act_stage_load(st, g.x, g.ntok, t0, c + 1, q8k, kSums);
-            if (wave_ok) {
-                wchunk_load<T>(w1, g.m, arow, arow_ok, orow, c + 1, kq, nb_of(c + 1));
-            }
+            act_stage_load(st, g.x, g.ntok, t0, c + 1);
+            if (wave_ok) wchunk_load(w1, g.m, arow, arow_ok, orow, c + 1, kq);
         }
-        if (wave_ok) {
-            wchunk_compute<T>(w0, L, a, lut16, nb_of(c));
-        }
+        if (wave_ok) wchunk_compute(w0, L, a);
         if (c + 1 >= nc) break;
-        // chunk c + 1 (weights in w1/v1)
+        // chunk c + 1 (weights in w1)
         __syncthreads();
-        act_stage_store(st, L, q8k, kSums);
+        act_stage_store(st, L);
         __syncthreads();
         if (c + 2 < nc) {
-            act_stage_load(st, g.x, g.ntok, t0, c + 2, q8k, kSums);
-            if (wave_ok) {
-                wchunk_load<T>(w0, g.m, arow, arow_ok, orow, c + 2, kq, nb_of(c + 2));
-            }
+            act_stage_load(st, g.x, g.ntok, t0, c + 2);
+            if (wave_ok) wchunk_load(w0, g.m, arow, arow_ok, orow, c + 2, kq);
         }
-        if (wave_ok) {
-            wchunk_compute<T>(w1, L, a, lut16, nb_of(c + 1));
-        }
+        if (wave_ok) wchunk_compute(w1, L, a);
     }
     if (!wave_ok) return;
 #pragma unroll
@@ -1281,6 +1061,361 @@ __global__ __launch_bounds__(64 * W) void k_mmx(MmArgs g) {
                 } else {
                     *o = gv / (1.0f + ref_expf_s(-gv)) * v;  // src/kernels_f32.cpp:287-289
                 }
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------- the GEMM of the 32-value formats and TQ2_0
+
+// Tokens are the MFMA's rows (A), weight rows its columns (B): v_mfma_i32_32x32x32_i8 takes one 32-value
+// block a step (K = 32), and D holds, in lane l, weight row l % 32 and tokens 8 (i / 4) + 4 (l / 32) + i % 4.
+// A wave computes 32 weight rows x 8 TG tokens (the first 8 TG of D's rows), a workgroup four such row
+// groups over the same tokens, so a lane has one weight row: its scales are one conversion a block, and
+// the tokens' scales come as broadcast float4 reads.
+//
+// What bounds it is the float term: the reference adds (float)dot * d_w * d_x a block and output
+// (src/quant.cpp:445-482), four vector operations.  Here the int32 dot comes out of the MFMA on top of
+// 0x4B400000, the bits of 1.5 * 2^23: read as a float that is 1.5 * 2^23 + dot exactly (|dot| < 2^22), and
+//   fma(that, d_w, -1.5 * 2^23 * d_w) = RN(dot * d_w)
+// since the product with a half's 11 bits and the constant's 13 are exact inside the fma: the conversion
+// and the first product in one operation.  (A scale that is not finite takes the two-step form.)  The
+// 4- and 5-bit values enter scaled by 16 or 8, which puts them at the top of the int8 with a shift and an
+// xor; d_w takes the factor back, exactly.
+//
+// Q8_0 6144 x 2048, 512 tokens: 44 us, 0.29 Pop/s (the form before, 16 x 16 MFMAs with a conversion and three
+// scale reads an output, 82 us).  55% of the vector unit's issue slots are full: 187 registers hold two
+// workgroups a compute unit, whose 768 tiles are one and a half rounds.  A few tokens are bound by the chunk's
+// latency instead (1.7 us a chunk and workgroup).
+constexpr int kMgWaves = 4;
+
+// Store, add, or gate/up pair of up to kMgMats matrices of one format over the same rows of activations.
+constexpr int kMgMats = 4;
+struct MgArgs {
+    MmArgs a;            // the activations and, for the pair, m2 and the gate
+    Packed m[kMgMats];
+    float* out[kMgMats];
+    int ostride[kMgMats];
+    int tiles[kMgMats];  // workgroup row tiles of each
+};
+
+constexpr float kMgMagic = 12582912.0f;  // 1.5 * 2^23
+template <uint32_t T>
+__host__ __device__ constexpr float mg_unscale() { return T == kQ4_0 ? 0.0625f : T == kQ5_0 ? 0.125f : 1.0f; }
+
+// A wave's weights of a 256-value chunk: its 32 rows, kP 16-byte pieces a row.  They are loaded with
+// consecutive lanes on consecutive pieces and go to the wave's own LDS, from where a lane reads its row's
+// fragments: read straight into fragment order, a load touches 32 rows, and the 64 cycles it then takes
+// in the address unit bounded the kernel.  Row r's piece p is at r * kP + (p ^ mg_swz(r)): the rows that
+// share banks differ in their pieces.  The block scales (Q4_1: and offsets) and Q5_0's fifth bits follow.
+template <uint32_t T>
+__host__ __device__ constexpr int mg_pieces() { return T == kQ8_0 ? 16 : T == kTQ2_0 ? 4 : 8; }
+template <uint32_t T>
+__device__ __forceinline__ int mg_swz(int r) { return T == kQ8_0 ? r & 15 : T == kTQ2_0 ? (r >> 2) & 3 : (r >> 1) & 7; }
+
+template <uint32_t T>
+struct MgRegs {  // in flight: a lane's pieces k * 64 + lane, and its piece of the scales
+    v4u q[mg_pieces<T>() / 2];
+    uint4 e, f;
+};
+template <uint32_t T>
+struct MgWave {
+    v4u q[32 * mg_pieces<T>()];
+    uint4 e[T == kTQ2_0 ? 1 : 64];   // row r's 8 fp16 scales at r; Q4_1: its offsets at 32 + r
+    uint4 f[T == kQ5_0 ? 64 : 1];    // Q5_0: row r's 8 words of fifth bits at 2 r, 2 r + 1
+    float d[T == kTQ2_0 ? 32 : 1];   // TQ2_0: row r's scale
+};
+
+// Chunk c of rows r0 .. r0 + 31 (rows past the matrix and pieces past the row: copies of the last).
+template <uint32_t T>
+__device__ __forceinline__ void mg_load(MgRegs<T>& w, const Packed& m, uint32_t r0, int c, int nb) {
+    constexpr int P = mg_pieces<T>();
+    const int lane = threadIdx.x & 63;
+    const uint32_t rmax = m.rows - 1, units = T == kTQ2_0 ? m.cols / 256 : m.cols / 32;
+    const int last = T == kQ8_0 ? 2 * nb - 1 : T == kTQ2_0 ? 3 : nb - 1;
+    auto row_of = [&](int r) -> size_t { return r0 + r <= rmax ? r0 + r : rmax; };
+#pragma unroll
+    for (int k = 0; k < P / 2; ++k) {
+        const int i = k * 64 + lane, r = i / P, p = i % P < last ? i % P : last;
+        const size_t blk = row_of(r) * units;
+        const uint8_t* base = T == kTQ2_0 ? m.p0 + (blk + c) * 64 : m.p0 + (blk + 8 * c) * (T == kQ8_0 ? 32 : 16);
+        w.q[k] = *gmem(reinterpret_cast<const v4u*>(base) + p);
+    }
+    if constexpr (T == kTQ2_0) {
+        w.e.x = gld<uint16_t>(m.p1, row_of(lane & 31) * units + c);
+    } else {
+        if (lane < 32 || T == kQ4_1) w.e = chunk_halves(lane < 32 ? m.p1 : m.p2, row_of(lane & 31) * units + 8 * c, nb);
+        if constexpr (T == kQ5_0) {
+            const uint32_t* qh = reinterpret_cast<const uint32_t*>(m.p2) + row_of(lane >> 1) * units + 8 * c;
+            uint32_t v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int j = 4 * (lane & 1) + k;
+                v[k] = gld<uint32_t>(qh, j < nb ? j : nb - 1);
+            }
+            w.f = make_uint4(v[0], v[1], v[2], v[3]);
+        }
+    }
+}
+// ... into the wave's LDS (its reads of the chunk before are done: a wave's LDS operations run in order).
+template <uint32_t T>
+__device__ __forceinline__ void mg_put(MgWave<T>& L, const MgRegs<T>& w) {
+    constexpr int P = mg_pieces<T>();
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int k = 0; k < P / 2; ++k) {
+        const int i = k * 64 + lane, r = i / P;
+        L.q[r * P + ((i % P) ^ mg_swz<T>(r))] = w.q[k];
+    }
+    if constexpr (T == kTQ2_0) {
+        if (lane < 32) L.d[lane] = h2f(static_cast<uint16_t>(w.e.x));
+    } else {
+        if (lane < 32 || T == kQ4_1) L.e[lane] = w.e;
+        if constexpr (T == kQ5_0) L.f[lane] = w.f;
+    }
+}
+
+// A lane's scales of a chunk (row l % 32).
+struct MgS {
+    uint4 sc, mn, qh[2];
+};
+template <uint32_t T>
+__device__ __forceinline__ MgS mg_scales(const MgWave<T>& L) {
+    const int r = threadIdx.x & 31;
+    MgS s{};
+    if constexpr (T != kTQ2_0) s.sc = L.e[r];
+    if constexpr (T == kQ4_1) s.mn = L.e[32 + r];
+    if constexpr (T == kQ5_0) {
+        s.qh[0] = L.f[2 * r];
+        s.qh[1] = L.f[2 * r + 1];
+    }
+    return s;
+}
+
+// The B operand of step jj for a lane (row l % 32, half h = l / 32 of the 32 values): 16 values as int8
+// (Q4_0: 16 (q - 8); Q4_1: q; Q5_0: 8 (q - 16); Q8_0; TQ2_0: code - 1).
+template <uint32_t T>
+__device__ __forceinline__ v4u mg_frag(const MgWave<T>& L, const MgS& sc, int jj, int h) {
+    const int r = threadIdx.x & 31;
+    const int p = T == kQ8_0 ? 2 * jj + h : T == kTQ2_0 ? 2 * (jj >> 2) + h : jj;
+    const v4u q = L.q[r * mg_pieces<T>() + (p ^ mg_swz<T>(r))];
+    if (T == kQ8_0) return q;
+    if (T == kQ4_0) return ((q << (h ? 0u : 4u)) & 0xF0F0F0F0u) ^ 0x80808080u;
+    if (T == kQ4_1) return (q >> (h ? 4u : 0u)) & 0x0F0F0F0Fu;
+    if (T == kQ5_0) {
+        const uint32_t bits = u4_word(sc.qh[jj >> 2], jj & 3) >> (16 * h);
+        v4u f = ((q >> (h ? 4u : 0u)) & 0x0F0F0F0Fu) << 3;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)  // four fifth bits to bit 7 of four bytes (24-bit product: no carries)
+            f[k] = (f[k] | ((__umul24((bits >> (4 * k)) & 0xFu, 0x00204081u) & 0x01010101u) << 7)) ^ 0x80808080u;
+        return f;
+    }
+    v4u f = (q >> (2u * (jj & 3))) & 0x03030303u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) f[k] = __builtin_amdgcn_perm(0u, 0x020100FFu, f[k]);  // byte code - 1, by table
+    return f;
+}
+
+__device__ __forceinline__ bool halves_not_finite(const uint4& v) {
+    auto hit = [](uint32_t w) { return ((w & 0x7C007C00u) + 0x04000400u) & 0x80008000u; };
+    return (hit(v.x) | hit(v.y) | hit(v.z) | hit(v.w)) != 0;
+}
+
+// Lane i of each 16-lane row's value in every lane of the row (a DPP operand of the instruction that uses it).
+template <int I>
+__device__ __forceinline__ float row_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + I, 0xF, 0xF, true));
+}
+// Calls f(integral_constant i) for i = 0 .. N - 1.
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<N, I + 1>(f);
+    }
+}
+
+template <uint32_t T, int TG, int NM>
+struct MgLds {
+    alignas(16) int8_t b[2][8 * TG][kBRow];
+    alignas(16) float xd[2][T == kTQ2_0 ? 1 : 8][8 * TG];   // [block][token]
+    alignas(16) float xs[2][T == kQ4_1 ? 8 : 1][8 * TG];    // Q4_1: d_x * sum
+    alignas(16) MgWave<T> w[kMgWaves][NM];
+};
+
+template <uint32_t T, int MODE, int TG>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_mg(MgArgs ga) {
+    constexpr int kTok = 8 * TG, NM = MODE == kMmPair ? 2 : 1;
+    __shared__ MgLds<T, TG, NM> L;
+    constexpr bool kSums = T == kQ4_1, q8k = T == kTQ2_0;
+    const MmArgs& g = ga.a;
+    int tile = blockIdx.x, ti = 0;
+    while (ti < kMgMats - 1 && tile >= ga.tiles[ti]) tile -= ga.tiles[ti++];
+    const Packed m = ga.m[ti];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5;
+    const uint32_t r0 = (static_cast<uint32_t>(tile) * kMgWaves + wave) * 32, rmax = m.rows - 1;
+    const uint32_t row = r0 + (lane & 31) <= rmax ? r0 + (lane & 31) : rmax;
+    const int t0 = blockIdx.y * kTok;
+    const bool lut16 = (m.flags & kFlagLut16) != 0;
+    const int nc = static_cast<int>((m.cols + kChunkCols - 1) / kChunkCols), nsub = static_cast<int>(m.cols / 32);
+    auto nb_of = [&](int c) { return nsub - 8 * c < 8 ? nsub - 8 * c : 8; };
+
+    // the workgroup's activations of a chunk, through registers: pieces of 16 bytes, and the scales
+    constexpr int kPieces = (kTok * 16 + kThreads - 1) / kThreads;
+    uint4 aq[kPieces];
+    float ad = 0.0f, as = 0.0f;
+    auto tokc = [&](int t) -> size_t { return static_cast<size_t>(t0 + t < g.ntok ? t0 + t : g.ntok - 1); };
+    auto act_load = [&](int c) {
+#pragma unroll
+        for (int k = 0; k < kPieces; ++k) {
+            const int i = k * kThreads + tid;
+            if (kTok * 16 % kThreads == 0 || i < kTok * 16) aq[k] = ld16(reinterpret_cast<const uint8_t*>(g.x.qs) + tokc(i >> 4) * g.x.stride + c * kChunkCols + (i & 15) * 16);
+        }
+        if (q8k) {
+            if (tid < kTok) ad = gld<float>(g.x.d, tokc(tid) * (g.x.stride / 32) + c);
+        } else if (tid < kTok * 8) {
+            ad = gld<float>(g.x.d, tokc(tid >> 3) * (g.x.stride / 32) + c * 8 + (tid & 7));
+            if (kSums) as = ad * static_cast<float>(gld<int32_t>(g.x.bs, tokc(tid >> 3) * (g.x.stride / 16) + c * 8 + (tid & 7)));
+        }
+    };
+    auto act_store = [&](int s) {
+#pragma unroll
+        for (int k = 0; k < kPieces; ++k) {
+            const int i = k * kThreads + tid;
+            if (kTok * 16 % kThreads == 0 || i < kTok * 16) *reinterpret_cast<uint4*>(&L.b[s][i >> 4][(i & 15) * 16]) = aq[k];
+        }
+        if (q8k) {
+            if (tid < kTok) L.xd[s][0][tid] = ad;
+        } else if (tid < kTok * 8) {
+            L.xd[s][tid & 7][tid >> 3] = ad;
+            if (kSums) L.xs[s][tid & 7][tid >> 3] = as;
+        }
+    };
+
+    if (MODE == kMmPair) exp_tab_fill();  // ordered before the epilogue by the loop's barriers
+    MgRegs<T> w[NM];
+    const Packed mm[2] = {m, NM == 2 ? g.m2 : m};
+    act_load(0);
+#pragma unroll
+    for (int n = 0; n < NM; ++n) mg_load<T>(w[n], mm[n], r0, 0, nb_of(0));
+#pragma unroll
+    for (int n = 0; n < NM; ++n) mg_put<T>(L.w[wave][n], w[n]);
+    act_store(0);
+    __syncthreads();
+    float acc[NM][4 * TG];
+#pragma unroll
+    for (int n = 0; n < NM; ++n)
+#pragma unroll
+        for (int i = 0; i < 4 * TG; ++i) acc[n][i] = 0.0f;
+    v16i magic;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) magic[i] = q8k ? 0 : 0x4B400000;
+    if (!q8k) asm volatile("" : "+v"(magic));  // held in registers, not rebuilt for every MFMA
+    const int atok = (lane & 31) & (kTok - 1);  // A's row (rows past the tile's tokens: copies, never read)
+    // the token of this lane's half's output i = l % 16: a 16-lane row holds its half's token scales, one
+    // small read a block, and each product takes its own by DPP (as float4 broadcasts, 32 128-bit reads a
+    // chunk, they bounded the kernel)
+    const int stok = 8 * (((lane & 15) >> 2) & (TG - 1)) + 4 * h + (lane & 3);
+
+    for (int c = 0; c < nc; ++c) {
+        const int s = c & 1, nb = nb_of(c);
+        if (c + 1 < nc) {
+            act_load(c + 1);
+#pragma unroll
+            for (int n = 0; n < NM; ++n) mg_load<T>(w[n], mm[n], r0, c + 1, nb_of(c + 1));
+        }
+        MgS sc[NM];
+#pragma unroll
+        for (int n = 0; n < NM; ++n) sc[n] = mg_scales<T>(L.w[wave][n]);
+        auto afrag = [&](int jj) { return *reinterpret_cast<const v4u*>(&L.b[s][atok][jj * 32 + 16 * h]); };
+        if constexpr (T == kTQ2_0) {
+            v16i d[NM];
+#pragma unroll
+            for (int n = 0; n < NM; ++n) d[n] = magic;
+#pragma unroll
+            for (int jj = 0; jj < 8; ++jj) {  // the block's int32 sum over its 8 steps, exact
+                const v4u a = afrag(jj);
+#pragma unroll
+                for (int n = 0; n < NM; ++n) d[n] = mfma32(a, mg_frag<T>(L.w[wave][n], sc[n], jj, h), d[n]);
+            }
+            float wd[NM];
+#pragma unroll
+            for (int n = 0; n < NM; ++n) wd[n] = L.w[wave][n].d[lane & 31];
+            const float xv = L.xd[s][0][stok];
+            static_for<4 * TG>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const float xd = row_bcast<i>(xv);
+#pragma unroll
+                for (int n = 0; n < NM; ++n) {
+                    const float v = static_cast<float>(d[n][i]);
+                    acc[n][i] += lut16 ? v * wd[n] * xd : xd * wd[n] * v;  // src/quant.cpp:789-802 / :580-596
+                }
+            });
+        } else {
+            bool odd = nb < 8;
+#pragma unroll
+            for (int n = 0; n < NM; ++n) odd = odd || halves_not_finite(sc[n].sc);
+            auto dots = [&](int jj, int n) { return mfma32(afrag(jj), mg_frag<T>(L.w[wave][n], sc[n], jj, h), magic); };
+            auto half_at = [](const uint4& v, int jj) {
+                const uint32_t word = u4_word(v, jj >> 1);
+                return h2f(static_cast<uint16_t>((jj & 1) ? (word >> 16) : (word & 0xFFFF)));
+            };
+            auto terms = [&](auto fast, int jj, int n, const v16i& d) {
+                const float wd = half_at(sc[n].sc, jj) * mg_unscale<T>(), cw = -kMgMagic * wd;
+                const float wm = kSums ? half_at(sc[n].mn, jj) : 0.0f;
+                const float xv = L.xd[s][jj][stok], sv = kSums ? L.xs[s][jj][stok] : 0.0f;
+                static_for<4 * TG>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const float f = __int_as_float(d[i]);
+                    const float p = decltype(fast)::value ? __builtin_fmaf(f, wd, cw) : (f - kMgMagic) * wd;
+                    if constexpr (kSums) acc[n][i] += row_bcast<i>(xv) * p + row_bcast<i>(sv) * wm;
+                    else acc[n][i] += row_bcast<i>(xv) * p;
+                });
+            };
+            if (__builtin_amdgcn_ballot_w64(odd) == 0) {  // the next dots under these terms
+                v16i d[2];
+                d[0] = dots(0, 0);
+#pragma unroll
+                for (int u = 0; u < 8 * NM; ++u) {
+                    if (u + 1 < 8 * NM) d[(u + 1) & 1] = dots((u + 1) / NM, (u + 1) % NM);
+                    terms(std::true_type{}, u / NM, u % NM, d[u & 1]);
+                }
+            } else {  // the row ends inside the chunk, or a scale is not finite
+#pragma unroll
+                for (int jj = 0; jj < 8; ++jj) {
+                    if (jj >= nb) break;  // past the row: no term
+#pragma unroll
+                    for (int n = 0; n < NM; ++n) terms(std::false_type{}, jj, n, dots(jj, n));
+                }
+            }
+        }
+        if (c + 1 < nc) {
+            act_store(s ^ 1);
+#pragma unroll
+            for (int n = 0; n < NM; ++n) mg_put<T>(L.w[wave][n], w[n]);
+        }
+        __syncthreads();
+    }
+    if (r0 + (lane & 31) > rmax) return;
+#pragma unroll
+    for (int i = 0; i < 4 * TG; ++i) {
+        const int t = t0 + 8 * (i >> 2) + 4 * h + (i & 3);
+        if (t >= g.ntok) continue;
+        float* o = ga.out[ti] + static_cast<size_t>(t) * ga.ostride[ti] + row;
+        const float v = acc[0][i];
+        if (MODE == kMmStore) {
+            *o = v;
+        } else if (MODE == kMmAdd) {
+            *o = *o + v;  // h += proj (src/model.cpp:1111, :1162)
+        } else {
+            const float up = acc[NM - 1][i];
+            if (g.relu2) {
+                const float q = v > 0.0f ? v : 0.0f;
+                *o = q * q * up;  // src/model.cpp:1134-1138
+            } else if (g.gelu) {
+                *o = gelu_mul(v, up);  // src/kernels_f32.cpp:291-296
+            } else {
+                *o = v / (1.0f + ref_expf_s(-v)) * up;  // src/kernels_f32.cpp:287-289
             }
         }
     }
@@ -2492,23 +2627,61 @@ static void mmx_launch(const MmArgs& g, hipStream_t s) {
     else hipLaunchKernelGGL((k_mmx<MODE, 1, 1, KM>), dim3(tiles(1)), dim3(64), 0, s, g);
 }
 
+// k_mg's tokens a workgroup.  A wider tile reads the weights fewer times and does an MFMA's full work (with 8
+// tokens three quarters of its rows are copies), but a launch is as long as its longest workgroup: 32 tokens
+// once that gives more workgroups than compute units, 16 once half as many, else 8.  Measured, in us at 32 / 16 /
+// 8 tokens (workgroups at 32): Q8_0 6144 x 2048, 512 tokens 45 / 51 / 78 (768); 4096 rows 28 / 34 / 48 (512);
+// Q4_0 pair of 3584 rows x 1024 30 / 36 / 50 (448); Q8_0 2048 x 6144 56 / 54 / 75 (256); Q4_0 1024 x 3584
+// 33 / 25 / 27 (128); TQ2_0 pair of 6912 x 2560, 64 tokens 19 / 17 / 20 (108); 3840 rows 11 / 10 / 9 (60);
+// Q4_0 pair of 3072 x 1024, 33 tokens 20 / 15 / 13 (48).
+template <uint32_t T, int MODE>
+static void mg_launch_t(MgArgs a, int n, hipStream_t s) {
+    int rt = 0;
+    for (int i = 0; i < kMgMats; ++i) {
+        a.tiles[i] = i < n ? static_cast<int>((a.m[i].rows + 32 * kMgWaves - 1) / (32 * kMgWaves)) : 0;
+        rt += a.tiles[i];
+    }
+    auto tt = [&](int tg) { return (a.a.ntok + 8 * tg - 1) / (8 * tg); };
+    const int tg = rt * tt(4) > kKqCus ? 4 : rt * tt(2) >= kKqCus / 2 ? 2 : 1;
+    const dim3 grid(rt, tt(tg));
+    if (tg == 4) hipLaunchKernelGGL((k_mg<T, MODE, 4>), grid, dim3(kThreads), 0, s, a);
+    else if (tg == 2) hipLaunchKernelGGL((k_mg<T, MODE, 2>), grid, dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL((k_mg<T, MODE, 1>), grid, dim3(kThreads), 0, s, a);
+}
+static bool mg_takes(uint32_t type) { return type == kQ4_0 || type == kQ4_1 || type == kQ5_0 || type == kQ8_0 || type == kTQ2_0; }
+// g, or with n > 1 the n GEMMs of g[] (one format and width, the same activations), as one launch.
+template <int MODE>
+static hipError_t mg_launch(const MmArgs* g, int n, hipStream_t s) {
+    MgArgs a{};
+    a.a = g[0];
+    for (int i = 0; i < n; ++i) {
+        a.m[i] = g[i].m;
+        a.out[i] = g[i].out;
+        a.ostride[i] = g[i].ostride;
+    }
+    switch (g[0].m.type) {
+        case kQ4_0: mg_launch_t<kQ4_0, MODE>(a, n, s); break;
+        case kQ4_1: mg_launch_t<kQ4_1, MODE>(a, n, s); break;
+        case kQ5_0: mg_launch_t<kQ5_0, MODE>(a, n, s); break;
+        case kQ8_0: mg_launch_t<kQ8_0, MODE>(a, n, s); break;
+        case kTQ2_0: mg_launch_t<kTQ2_0, MODE>(a, n, s); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 template <int MODE>
 static hipError_t mm_dispatch(const MmArgs& g, hipStream_t s) {
-    const int tok = 16 * (g.m.type == kQ4_K || g.m.type == kQ5_K || g.m.type == kQ6_K ? mm_groups<kQ4_K>() : mm_groups<kQ4_0>());
-    const dim3 grid((g.m.rows + kRowsPerWg - 1) / kRowsPerWg, (g.ntok + tok - 1) / tok);
+    const dim3 grid((g.m.rows + kRowsPerWg - 1) / kRowsPerWg, (g.ntok + kQ5Tok - 1) / kQ5Tok);
     // K-quants: the widest token tile (64, 32 or 16 tokens) that still gives a workgroup to every CU
     const int row_tiles = static_cast<int>((g.m.rows + 63) / 64);
     int kq_g = 4;
     while (kq_g > 1 && row_tiles * ((g.ntok + 16 * kq_g - 1) / (16 * kq_g)) < kKqCus) kq_g /= 2;
     const dim3 kq_grid(row_tiles, (g.ntok + 16 * kq_g - 1) / (16 * kq_g));
     switch (g.m.type) {
-        case kQ4_0: hipLaunchKernelGGL((k_mm<kQ4_0, MODE>), grid, dim3(kThreads), 0, s, g); break;
-        case kQ4_1: hipLaunchKernelGGL((k_mm<kQ4_1, MODE>), grid, dim3(kThreads), 0, s, g); break;
-        case kQ5_0: hipLaunchKernelGGL((k_mm<kQ5_0, MODE>), grid, dim3(kThreads), 0, s, g); break;
-        case kQ8_0: hipLaunchKernelGGL((k_mm<kQ8_0, MODE>), grid, dim3(kThreads), 0, s, g); break;
         case kQ5_K:
             if (g.qx != nullptr) mmx_launch<MODE, true>(g, s);
-            else hipLaunchKernelGGL((k_mm<kQ5_K, MODE>), grid, dim3(kThreads), 0, s, g);
+            else hipLaunchKernelGGL((k_mm<MODE>), grid, dim3(kThreads), 0, s, g);
             break;
         case kQ4_K:
             if (g.qx != nullptr) {
@@ -2528,7 +2701,6 @@ static hipError_t mm_dispatch(const MmArgs& g, hipStream_t s) {
             else if (kq_g == 2) hipLaunchKernelGGL((k_mmk<kQ6_K, MODE, 2>), kq_grid, dim3(kThreads), 0, s, g, g);
             else hipLaunchKernelGGL((k_mmk<kQ6_K, MODE, 1>), kq_grid, dim3(kThreads), 0, s, g, g);
             break;
-        case kTQ2_0: hipLaunchKernelGGL((k_mm<kTQ2_0, MODE>), grid, dim3(kThreads), 0, s, g); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -2540,14 +2712,25 @@ static bool pair_split() {
     return e != nullptr && std::string(e) == "1";
 }
 
+// Rows of whole 256-value chunks; the 32-value-block formats (k_mg) also take a partial last chunk.
+static bool mm_shape_ok(const MmArgs& g) {
+    const bool small_blocks = mg_takes(g.m.type) && g.m.type != kTQ2_0;
+    return (g.m.cols % kChunkCols == 0 || (small_blocks && g.m.cols % 32 == 0)) && g.x.stride % kChunkCols == 0 &&
+           static_cast<size_t>(g.x.stride) >= g.m.cols;
+}
+
 hipError_t launch_mm(const MmArgs& g, int mode, hipStream_t s) {
     if (g.ntok <= 0) return hipSuccess;
-    // rows of whole 256-value chunks; the 32-value-block formats (k_mm) also take a partial last chunk
-    const bool small_blocks = g.m.type == kQ4_0 || g.m.type == kQ4_1 || g.m.type == kQ5_0 || g.m.type == kQ8_0;
-    if ((g.m.cols % kChunkCols != 0 && !(small_blocks && g.m.cols % 32 == 0)) || g.x.stride % kChunkCols != 0 ||
-        static_cast<size_t>(g.x.stride) < g.m.cols)
-        return hipErrorInvalidValue;
+    if (!mm_shape_ok(g)) return hipErrorInvalidValue;
     if (mode == kMmPair && (g.m2.type != g.m.type || g.m2.rows != g.m.rows || g.m2.cols != g.m.cols)) return hipErrorInvalidValue;
+    if (mg_takes(g.m.type)) {
+        switch (mode) {
+            case kMmStore: return mg_launch<kMmStore>(&g, 1, s);
+            case kMmAdd: return mg_launch<kMmAdd>(&g, 1, s);
+            case kMmPair: return mg_launch<kMmPair>(&g, 1, s);
+            default: return hipErrorInvalidValue;
+        }
+    }
     switch (mode) {
         case kMmStore: return mm_dispatch<kMmStore>(g, s);
         case kMmAdd: return mm_dispatch<kMmAdd>(g, s);
@@ -2576,14 +2759,8 @@ hipError_t launch_mm(const MmArgs& g, int mode, hipStream_t s) {
     }
 }
 
-hipError_t launch_mm_two(const MmArgs& a, const MmArgs& b, hipStream_t s) {
-    if (a.ntok <= 0) return hipSuccess;
-    const bool fuse = a.m.type == kQ4_K && b.m.type == kQ4_K && a.m.cols == b.m.cols && a.qx == nullptr && b.qx == nullptr &&
-                      a.ntok == b.ntok && a.x.qs == b.x.qs && a.m.cols % kChunkCols == 0 && a.x.stride % kChunkCols == 0;
-    if (!fuse) {
-        const hipError_t e = launch_mm(a, kMmStore, s);
-        return e != hipSuccess ? e : launch_mm(b, kMmStore, s);
-    }
+// Two Q4_K store GEMMs of one activation and width (packed planes): one launch over both.
+static hipError_t mmk_two(const MmArgs& a, const MmArgs& b, hipStream_t s) {
     // the widest token tile that still gives a workgroup to every CU, over both matrices' row tiles
     const int row_tiles = static_cast<int>((a.m.rows + 63) / 64 + (b.m.rows + 63) / 64);
     int kq_g = 4;
@@ -2593,6 +2770,26 @@ hipError_t launch_mm_two(const MmArgs& a, const MmArgs& b, hipStream_t s) {
     else if (kq_g == 2) hipLaunchKernelGGL((k_mmk<kQ4_K, kMmStore, 2, true>), grid, dim3(kThreads), 0, s, a, b);
     else hipLaunchKernelGGL((k_mmk<kQ4_K, kMmStore, 1, true>), grid, dim3(kThreads), 0, s, a, b);
     return hipGetLastError();
+}
+
+hipError_t launch_mm_store(const MmArgs* g, int n, hipStream_t s) {
+    if (n <= 0 || g[0].ntok <= 0) return hipSuccess;
+    const MmArgs &a = g[0], &b = g[n > 1 ? 1 : 0];
+    auto alike = [&](const MmArgs& o) {
+        return o.m.type == a.m.type && o.m.cols == a.m.cols && o.ntok == a.ntok && o.x.qs == a.x.qs && o.x.stride == a.x.stride;
+    };
+    int k = 1;  // the first k GEMMs as one launch
+    if (mg_takes(a.m.type)) {
+        while (k < n && k < kMgMats && alike(g[k])) ++k;
+    } else if (n > 1 && a.m.type == kQ4_K && alike(b) && a.qx == nullptr && b.qx == nullptr) {
+        k = 2;
+    }
+    const bool shape_ok = mm_shape_ok(a);
+    hipError_t e = hipSuccess;
+    if (k == 1 || !shape_ok) e = launch_mm(a, kMmStore, s);
+    else if (mg_takes(a.m.type)) e = mg_launch<kMmStore>(g, k, s);
+    else e = mmk_two(a, b, s);
+    return e != hipSuccess ? e : launch_mm_store(g + k, n - k, s);
 }
 
 static bool mx_km(uint32_t type) { return type == kQ4_K || type == kQ5_K; }

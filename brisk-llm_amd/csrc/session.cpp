@@ -1315,16 +1315,15 @@ void Session::prefill_layers(size_t pos0, int T) {
             const DeviceMatrix* mats[4] = {&L.ssm_qkv, &L.ssm_gate, &L.ssm_alpha, &L.ssm_beta};
             float* outs[4] = {pre_sqkv_, pre_sz_, pre_sab_, pre_sab_ + heads};
             const int strides[4] = {qkv, inner, 2 * heads, 2 * heads};
-            const DeviceMatrix* quantised_for = nullptr;
-            for (int i = 0; i < 4; ++i) {  // attn_norm(h) quantised once per activation format
+            for (int i = 0, k; i < 4; i = k) {  // attn_norm(h) quantised once per activation format
                 const DeviceMatrix& m = *mats[i];
-                if (quantised_for == nullptr || takes_q8_k(m.p.type) != takes_q8_k(quantised_for->p.type) ||
-                    act_bits(m.p) != act_bits(quantised_for->p)) {
-                    prefill_quant(pre_h_, e, L.attn_norm, e, T, m);
-                    quantised_for = &m;
+                prefill_quant(pre_h_, e, L.attn_norm, e, T, m);
+                MmArgs run[4];
+                for (k = i; k < 4 && takes_q8_k(mats[k]->p.type) == takes_q8_k(m.p.type) && act_bits(mats[k]->p) == act_bits(m.p); ++k) {
+                    run[k - i] = g;
+                    run[k - i].m = mats[k]->p; set_mx(run[k - i], *mats[k]); run[k - i].out = outs[k]; run[k - i].ostride = strides[k];
                 }
-                g.m = m.p; set_mx(g, m); g.out = outs[i]; g.ostride = strides[i];
-                check(launch_mm(g, kMmStore, stream_), "prefill recurrence projections");
+                check(launch_mm_store(run, k - i, stream_), "prefill recurrence projections");
             }
             PreSsmArgs ps{};
             SsmArgs& sa = ps.s;
@@ -1339,12 +1338,11 @@ void Session::prefill_layers(size_t pos0, int T) {
             check(launch_mm(g, kMmAdd, stream_), "prefill ssm_out");
         } else if (qwen35()) {  // Qwen3.5's gated attention: each head's query rows, then its gate rows
             prefill_quant(pre_h_, e, L.attn_norm, e, T, L.q);
-            g.m = L.q.p; set_mx(g, L.q); g.out = pre_qg_; g.ostride = 2 * qd;
-            check(launch_mm(g, kMmStore, stream_), "prefill q");
-            g.m = L.k.p; set_mx(g, L.k); g.out = pre_k_; g.ostride = kvd;
-            check(launch_mm(g, kMmStore, stream_), "prefill k");
-            g.m = L.v.p; set_mx(g, L.v); g.out = pre_v_; g.ostride = kvd;
-            check(launch_mm(g, kMmStore, stream_), "prefill v");
+            MmArgs qkv[3] = {g, g, g};
+            qkv[0].m = L.q.p; set_mx(qkv[0], L.q); qkv[0].out = pre_qg_; qkv[0].ostride = 2 * qd;
+            qkv[1].m = L.k.p; set_mx(qkv[1], L.k); qkv[1].out = pre_k_; qkv[1].ostride = kvd;
+            qkv[2].m = L.v.p; set_mx(qkv[2], L.v); qkv[2].out = pre_v_; qkv[2].ostride = kvd;
+            check(launch_mm_store(qkv, 3, stream_), "prefill q, k, v");
             PrePlainArgs pp{};
             AttnArgs& aa = pp.a;
             aa.q = pre_qg_; aa.k = pre_k_; aa.v = pre_v_; aa.qnorm = L.q_norm; aa.knorm = L.k_norm;
@@ -1376,17 +1374,17 @@ void Session::prefill_layers(size_t pos0, int T) {
             const bool own_kv = L.kv_src == static_cast<int>(l);
             prefill_quant(pre_h_, e, L.attn_norm, e, T, L.q);
             g.m = L.q.p; set_mx(g, L.q); g.out = pre_q_; g.ostride = qdl;
-            if (own_kv) {  // Q and K in one launch where their formats allow
-                MmArgs gk = g;
+            MmArgs qkv[3] = {g, g, g};  // in one launch where their formats allow
+            int nqkv = 1;
+            if (own_kv) {
+                MmArgs& gk = qkv[nqkv++];
                 gk.m = L.k.p; set_mx(gk, L.k); gk.out = pre_k_; gk.ostride = kvdl;
-                check(launch_mm_two(g, gk, stream_), "prefill q, k");
                 if (!L.v_is_k) {
-                    g.m = L.v.p; set_mx(g, L.v); g.out = pre_v_; g.ostride = kvdl;
-                    check(launch_mm(g, kMmStore, stream_), "prefill v");
+                    MmArgs& gv = qkv[nqkv++];
+                    gv.m = L.v.p; set_mx(gv, L.v); gv.out = pre_v_; gv.ostride = kvdl;
                 }
-            } else {
-                check(launch_mm(g, kMmStore, stream_), "prefill q");
             }
+            check(launch_mm_store(qkv, nqkv, stream_), "prefill q, k, v");
             // norms, RoPE, cache rows, attention (:1020-1093)
             if (plain_attn_) {  // heads past 128 (or BRISK_HIP_ATTN=plain): the plain attention batched
                 PrePlainArgs pp{};
