@@ -687,7 +687,7 @@ __global__ void k_log1pf(const float* __restrict__ x, float* __restrict__ y, siz
 //   scores   (a workgroup per query head and 64 positions, a lane per position):
 //            dot_f32(q, k_p) * scale, 16 lane partials over i = j (mod 16) in order, then
 //            0 + lane 0 + ... + lane 15;
-//   values   (a wave per head and 64 output dimensions): the head's softmax (max,
+//   values   (a workgroup per head and 64 output dimensions): the head's softmax (max,
 //            e_p = expf(s_p - max), their sum in double, w_p = e_p * (float)(1 / sum)), then
 //            for each output dimension 0 + w_0 v_0 + w_1 v_1 + ... in position order.
 // A sliding layer's token sees positions [L - window, L) (src/model.cpp:1084-1085).
@@ -766,45 +766,94 @@ __global__ __launch_bounds__(64) void k_plain_scores(AttnArgs g) {
     g.gsc[static_cast<size_t>(h) * g.ctx + p] = sum * g.scale;
 }
 
-// A wave per (head, 64 output dimensions): the head's softmax (each wave of the head computes the
-// same weights: max, e_p = expf(s_p - max), their double sum, e_p * (float)(1 / sum)), held in LDS
-// when the window fits it and recomputed per position otherwise; then a lane per output dimension
-// sums w_p v_p[d] in position order, its loads issued 32 positions at a time.  Qwen3.5's sigmoid
-// gate (src/model.cpp:1102-1108) is applied to the sums.
-__global__ __launch_bounds__(64) void k_plain_values(AttnArgs g) {
+// A workgroup per (head, 64 output dimensions): the head's softmax (each workgroup of the head computes the
+// same weights: max, e_p = expf(s_p - max), their double sum, e_p * (float)(1 / sum)), the e_p held in LDS
+// when the window fits it and recomputed per position otherwise; then the values.
+//
+// An output dimension is one chain of n adds in position order, and a decode step has only heads x
+// head_dim / 64 workgroups, so the chain is what bounds the kernel and nothing else may be on it: waves
+// 1 .. 6 read the value rows (a 16-byte piece a thread, coalesced, kVAhead batches of kVRows positions ahead)
+// and write w_p v_p to LDS as floats, and wave 0, a lane a dimension, only reads and adds them, a batch
+// behind.  With one wave that loaded, converted, multiplied and added, 701 positions of a 256-wide head took
+// 28 us (22 round trips to memory and 60 cycles a position); now 7.8 us.  Qwen3.5's sigmoid gate
+// (src/model.cpp:1102-1108) is applied to the sums.
+constexpr int kVWaves = 6, kVRows = 8 * kVWaves, kVAhead = 4;
+constexpr int kVThreads = 64 * (kVWaves + 1);
+__global__ __launch_bounds__(kVThreads) void k_plain_values(AttnArgs g) {
     __shared__ float wl[kPlainLdsW];
-    const int h = blockIdx.x, hd = g.head_dim, hpk = g.heads / g.kv_heads, kv = h / hpk, lane = threadIdx.x;
-    const int L = *g.pos + 1, start = plain_start(g, L), n = L - start;
+    __shared__ alignas(16) float prod[2][kVRows][64];
+    __shared__ float red[kVWaves + 1];
+    const int h = blockIdx.x, hd = g.head_dim, hpk = g.heads / g.kv_heads, kv = h / hpk, tid = threadIdx.x, wave = tid >> 6,
+              lane = tid & 63;
+    const int L = *g.pos + 1, start = plain_start(g, L), n = L - start, nb = (n + kVRows - 1) / kVRows;
     const float* sc = g.gsc + static_cast<size_t>(h) * g.ctx + start;
+    const int d0 = static_cast<int>(blockIdx.y) * 64;
+    // a thread of waves 1 ..: dimensions d0 + 8 piece .. + 7 of each batch's position r (pieces past the head: the first)
+    const int r = (tid - 64) >> 3, piece = tid & 7;
+    const uint16_t* vrow = g.vcache + (static_cast<size_t>(kv) * g.ctx + start) * hd + (d0 + 8 * piece < hd ? d0 + 8 * piece : d0);
+    auto load = [&](int b) {
+        const int p = b * kVRows + r;
+        return *reinterpret_cast<const uint4*>(vrow + static_cast<size_t>(p < n ? p : n - 1) * hd);
+    };
+    uint4 q[kVAhead];
+    if (wave != 0) {
+#pragma unroll
+        for (int u = 0; u < kVAhead; ++u) q[u] = load(u);
+    }
+    exp_tab_fill();
     float m = -INFINITY;
-    for (int p = lane; p < n; p += 64) m = fmaxf(m, sc[p]);
+    for (int p = tid; p < n; p += kVThreads) m = fmaxf(m, sc[p]);
     m = wave_max(m);
-    const bool in_lds = n <= kPlainLdsW;
-    double part = 0.0;
-    for (int p = lane; p < n; p += 64) {
-        const float e = ref_expf(sc[p] - m);
-        if (in_lds) wl[p] = e;
-        part += static_cast<double>(e);
-    }
-    const float scale = static_cast<float>(1.0 / wave_sum(part));
-    if (in_lds)
-        for (int p = lane; p < n; p += 64) wl[p] = wl[p] * scale;
+    if (lane == 0) red[wave] = m;
     __syncthreads();
-    const int d = static_cast<int>(blockIdx.y) * 64 + lane;
-    if (d >= hd) return;
-    const uint16_t* vv = g.vcache + static_cast<size_t>(kv) * g.ctx * hd + static_cast<size_t>(start) * hd + d;
-    auto weight = [&](int p) { return in_lds ? wl[p] : ref_expf(sc[p] - m) * scale; };
-    constexpr int kB = 32;
-    float a = 0.0f;
-    int p = 0;
-    for (; p + kB <= n; p += kB) {  // loads first, then the adds in position order
-        float vf[kB];
 #pragma unroll
-        for (int u = 0; u < kB; ++u) vf[u] = h2f(vv[static_cast<size_t>(p + u) * hd]);
-#pragma unroll
-        for (int u = 0; u < kB; ++u) a += weight(p + u) * vf[u];
+    for (int k = 0; k <= kVWaves; ++k) m = fmaxf(m, red[k]);
+    const bool in_lds = n <= kPlainLdsW;
+    if (in_lds) {
+        for (int p = tid; p < n; p += kVThreads) wl[p] = ref_expf_s(sc[p] - m);
+        __syncthreads();
     }
-    for (; p < n; ++p) a += weight(p) * h2f(vv[static_cast<size_t>(p) * hd]);
+    double part = 0.0;  // a lane's e_p, p = lane (mod 64), in order
+    for (int p = lane; p < n; p += 64) part += static_cast<double>(in_lds ? wl[p] : ref_expf_s(sc[p] - m));
+    const float scale = static_cast<float>(1.0 / wave_sum(part));
+    float a = 0.0f;
+    for (int b0 = 0; b0 < nb; b0 += kVAhead) {
+#pragma unroll
+        for (int u = 0; u < kVAhead; ++u) {
+            const int b = b0 + u;
+            if (b >= nb) break;
+            if (wave != 0) {
+                const int p = b * kVRows + r;
+                if (p < n) {
+                    const float w = (in_lds ? wl[p] : ref_expf_s(sc[p] - m)) * scale;
+                    const uint32_t vw[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
+                    float t[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) t[k] = w * h2f(static_cast<uint16_t>((k & 1) ? vw[k >> 1] >> 16 : vw[k >> 1] & 0xFFFF));
+                    float4* o = reinterpret_cast<float4*>(&prod[b & 1][r][8 * piece]);
+                    o[0] = make_float4(t[0], t[1], t[2], t[3]);
+                    o[1] = make_float4(t[4], t[5], t[6], t[7]);
+                }
+                q[u] = load(b + kVAhead);
+            }
+            __syncthreads();  // batch b is written, and wave 0 has added b - 1, whose buffer b + 1 takes
+            if (wave == 0) {
+                const float(*row)[64] = prod[b & 1];
+                const int c = n - b * kVRows;
+                if (c >= kVRows) {
+                    float t[kVRows];  // every read before the adds
+#pragma unroll
+                    for (int k = 0; k < kVRows; ++k) t[k] = row[k][lane];
+#pragma unroll
+                    for (int k = 0; k < kVRows; ++k) a += t[k];
+                } else {
+                    for (int k = 0; k < c; ++k) a += row[k][lane];
+                }
+            }
+        }
+    }
+    const int d = d0 + lane;
+    if (wave != 0 || d >= hd) return;
     if (g.gate != nullptr) a = a * (1.0f / (1.0f + ref_expf(-g.gate[static_cast<size_t>(h) * g.gate_stride + d])));
     g.out[h * hd + d] = a;
 }
@@ -1165,7 +1214,7 @@ hipError_t launch_attention_plain(const AttnArgs& g, hipStream_t s) {
     hipLaunchKernelGGL(k_plain_prologue, dim3(static_cast<unsigned>(g.heads + (g.no_kv ? 0 : g.kv_heads))), dim3(64), 0, s, g);
     hipLaunchKernelGGL(k_plain_scores, dim3(static_cast<unsigned>(g.heads), pos_blocks), dim3(64), 0, s, g);
     hipLaunchKernelGGL(k_plain_values, dim3(static_cast<unsigned>(g.heads), static_cast<unsigned>(g.head_dim / 64 + (g.head_dim % 64 != 0))),
-                       dim3(64), 0, s, g);
+                       dim3(kVThreads), 0, s, g);
     return hipGetLastError();
 }
 

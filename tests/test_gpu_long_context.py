@@ -91,6 +91,30 @@ def test_long_plain_attention(n_pos):
         o.close()
 
 
+@pytest.mark.parametrize("name", ["tiny-gemma3", "tiny-qwen3-long"])
+def test_plain_attention_value_batches(name):
+    """The plain attention's value sums go by batches of 48 positions, four read ahead: one token decoded
+    after contexts that end around a batch and around the read-ahead, bit-identical to the oracle."""
+    import os
+    f, cfg, table = model.load(synth.model_path(name))
+    os.environ["BRISK_HIP_ATTN"] = "plain"
+    try:
+        s = HipSession((f, cfg, table), max_context=320)
+    finally:
+        del os.environ["BRISK_HIP_ATTN"]
+    with s:
+        o = pyoracle.Oracle(cfg, table, 320)
+        prompt = synth.prompt_ids(300, cfg.vocab, seed=4)
+        for n in (0, 1, 46, 47, 48, 94, 95, 96, 191, 192, 239, 240, 287):
+            for h in (s, o):
+                h.rollback(0)
+                if n > 0:
+                    h.eval(prompt[:n])
+            got, want = s.eval([23]), o.eval([23])
+            np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32), err_msg=f"{name} after {n} positions")
+        o.close()
+
+
 @pytest.mark.slow
 def test_qwen3_1_7b_at_4096():
     """configs[3] at full size: Qwen3-1.7B-shape Q8_0, 4096 pre-filled positions, then decode."""
