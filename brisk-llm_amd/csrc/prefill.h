@@ -90,7 +90,7 @@ constexpr bool pre_attn_rows_fits(int head_dim, int L) {
 
 hipError_t launch_mm(const MmArgs& g, int mode, hipStream_t s);
 // The n store GEMMs g[] of one activation, in as few launches as their formats allow: up to four of one
-// 32-value format or TQ2_0 and one width, two packed-plane Q4_K of one width, else launch_mm of each.
+// 32-value format, TQ2_0 or packed-plane Q4_K and of one width share one, the others take launch_mm each.
 hipError_t launch_mm_store(const MmArgs* g, int n, hipStream_t s);
 // The GEMMs take rows whose length is a multiple of this many values (one staged chunk).
 constexpr int kMmChunkCols = 256;

@@ -421,9 +421,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 2))
     }
 }
 
-// ---------------------------------------------------------------- the K-quant GEMM, staged through LDS
+// ---------------------------------------------------------------- the packed Q6_K GEMM, staged through LDS
 
-// Q4_K / Q6_K (one 256-value super-block a row per chunk).  A workgroup of 4
+// Q6_K without expanded planes (one 256-value super-block a row per chunk).  A workgroup of 4
 // waves computes 64 rows x 32 tokens; wave w owns rows 16 w .. + 15 for the
 // 32 tokens (2 groups of 16).  Per chunk every operand -- the 64 rows' weight
 // planes and the 32 tokens' int8 values, bsums and scales -- is copied global
@@ -437,13 +437,12 @@ constexpr int kKqCus = 256;  // MI355X compute units (the tile choice aims at a 
 // tokens a workgroup: 16 G (G token groups share each weight fragment's decode); the
 // launcher takes the largest G that still gives a workgroup to every CU
 
-template <uint32_t T>
 struct KqStage {
-    alignas(16) uint8_t w0[64 * 128];                  // Q4_K nibbles / Q6_K ql: row r piece p at slot r * 8 + (p ^ (r & 7))
-    alignas(16) uint8_t wk[T == kQ4_K ? 2048 : 4096];  // Q4_K: p1 [64][16] then p2 [64][16]; Q6_K: qh, row r piece p at r * 4 + (p ^ (r & 3))
-    alignas(16) uint32_t wm[T == kQ6_K ? 384 : 1];     // Q6_K: the 20-byte meta of row r at dwords 5 r .. 5 r + 4
-    alignas(16) int8_t x[kKqTokMax * 256];             // token t piece p at slot t * 16 + (p ^ (t & 15))
-    alignas(16) float xd[64];                          // Q8_K scale of token t (lanes 32..63: a copy)
+    alignas(16) uint8_t w0[64 * 128];         // ql: row r piece p at slot r * 8 + (p ^ (r & 7))
+    alignas(16) uint8_t wk[4096];             // qh: row r piece p at r * 4 + (p ^ (r & 3))
+    alignas(16) uint32_t wm[384];             // the 20-byte meta of row r at dwords 5 r .. 5 r + 4
+    alignas(16) int8_t x[kKqTokMax * 256];    // token t piece p at slot t * 16 + (p ^ (t & 15))
+    alignas(16) float xd[64];                 // Q8_K scale of token t (lanes 32..63: a copy)
 };
 
 __device__ __forceinline__ void dma16(const void* src, void* lds_wave_base) {
@@ -455,8 +454,8 @@ __device__ __forceinline__ void dma4(const void* src, void* lds_wave_base) {
 
 // Copies chunk c of rows r0 .. r0 + 63 and tokens t0 .. t0 + 31 into the stage
 // (rows and tokens past the ends re-read the last one; their outputs are not stored).
-template <uint32_t T, int G>
-__device__ __forceinline__ void kq_copy(KqStage<T>& st, const Packed& m, const ActPlanar& x, int ntok, uint32_t r0, int t0, int c) {
+template <int G>
+__device__ __forceinline__ void kq_copy(KqStage& st, const Packed& m, const ActPlanar& x, int ntok, uint32_t r0, int t0, int c) {
     const int tid = threadIdx.x, wave = tid >> 6, wave_first = tid & ~63;
     const uint32_t nsb = m.cols / 256, rmax = m.rows - 1;
     auto rowc = [&](int r) -> size_t {
@@ -469,21 +468,16 @@ __device__ __forceinline__ void kq_copy(KqStage<T>& st, const Packed& m, const A
         const int slot = k * kThreads + tid, r = slot >> 3, p = (slot & 7) ^ (r & 7);
         dma16(m.p0 + rowc(r) * 128 + p * 16, st.w0 + (k * kThreads + wave_first) * 16);
     }
-    if (T == kQ4_K) {  // wave 0: the p1 rows, wave 1: the p2 rows
-        if (wave < 2) {
-            const int r = tid & 63;
-            dma16((wave ? m.p2 : m.p1) + rowc(r) * 16, st.wk + wave_first * 16);
-        }
-    } else {  // qh: 64 rows x 4 pieces; meta: 320 dwords
+    {  // qh: 64 rows x 4 pieces; meta: 320 dwords
         const int r = tid >> 2, p = (tid & 3) ^ (r & 3);
         dma16(m.p1 + rowc(r) * 64 + p * 16, st.wk + wave_first * 16);
+    }
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int slot = k * kThreads + tid;
-            if (slot < 384) {  // waves of slots 320..383 copy row 63's meta again into the spare
-                const int sl = slot < 320 ? slot : 319, r2 = sl / 5, j = sl - r2 * 5;
-                dma4(m.p2 + rowc(r2) * 20 + j * 4, st.wm + k * kThreads + wave_first);
-            }
+    for (int k = 0; k < 2; ++k) {
+        const int slot = k * kThreads + tid;
+        if (slot < 384) {  // waves of slots 320..383 copy row 63's meta again into the spare
+            const int sl = slot < 320 ? slot : 319, r2 = sl / 5, j = sl - r2 * 5;
+            dma4(m.p2 + rowc(r2) * 20 + j * 4, st.wm + k * kThreads + wave_first);
         }
     }
     const size_t ds = x.stride / 32;
@@ -524,57 +518,11 @@ __device__ __forceinline__ uint4 ds128(uint32_t a) {
     return make_uint4(r.x, r.y, r.z, r.w);
 }
 
-// Q4_K with the scales folded into the MFMAs.  For sub-block j of a row,
-// weighted = sum_j sc_j dot_j and offsets = sum_j mn_j pair_j (dot_q4_k_q8_k,
-// src/quant.cpp:500-521) are exact integers; with sc_j = lo_j + 8 hi_j (3-bit
-// digits) and q in 0..15, q lo_j and q hi_j fit int8, so
-//   weighted = A_lo + 8 A_hi,  A_lo = sum_k (q_k lo_j(k)) x_k,  A_hi likewise,
-//   offsets  = sum_k mn_j(k) x_k   (pair_j is the sum of sub-block j's x),
-// three int32 MFMA chains over the super-block, with no per-sub-block integer
-// epilogue.  The float term per super-block is the reference's.
-// The MFMA is v_mfma_i32_16x16x64_i8 (measured at 2.5 POP/s on register operands,
-// against 4.2 for v_mfma_i32_32x32x32_i8: brisk_hip_mfma_rate): lane l
-// holds 16 consecutive k of A row l % 16 and of B column l % 16, k = 16 (l / 16)
-// .. + 15 of the 64, so lanes 0..31 are sub-block 2 s and lanes 32..63
-// sub-block 2 s + 1 of step s, and each lane's digit is its own sub-block's.
+// v_mfma_i32_16x16x64_i8 (measured at 2.5 POP/s on register operands, against 4.2 for
+// v_mfma_i32_32x32x32_i8: brisk_hip_mfma_rate): lane l holds 16 consecutive k of A row l % 16 and of B
+// column l % 16, k = 16 (l / 16) .. + 15 of the 64.
 __device__ __forceinline__ v4i mfma64(const v4u& a, const v4u& b, v4i c) {
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, a), __builtin_bit_cast(v4i, b), c, 0, 0, 0);
-}
-
-// LDS addresses of a Q4_K stage's parts: the nibble rows, the {d, dmin, scales} and decoded
-// scale/min rows (wk, then wk + 1024), the activations and their scales.
-struct KqBases {
-    uint32_t w0, wk, x, xd;
-};
-__device__ __forceinline__ KqBases kq_bases(uint32_t base) {
-    return KqBases{base + static_cast<uint32_t>(offsetof(KqStage<kQ4_K>, w0)), base + static_cast<uint32_t>(offsetof(KqStage<kQ4_K>, wk)),
-                   base + static_cast<uint32_t>(offsetof(KqStage<kQ4_K>, x)), base + static_cast<uint32_t>(offsetof(KqStage<kQ4_K>, xd))};
-}
-
-// Fragments read by kq_f64_issue; kq_f64_wait ties each as one 128-bit operand,
-// so no copy of a fragment register can be placed before the wait.
-struct KqF64 {
-    v4u a, b0, b1, b2, b3;  // b0 .. b(G-1) used
-};
-template <int G>
-__device__ __forceinline__ KqF64 kq_f64_issue(const KqBases& b, int s, int ar, int tl, int l16) {
-    KqF64 f;
-    const int pa = 2 * s + (l16 & 1);  // Q4_K: 32 bytes of nibbles a sub-block pair, low then high
-    f.a = ds128v(b.w0 + (ar * 8 + (pa ^ (ar & 7))) * 16);
-    const int pb = 4 * s + l16;
-    auto bfrag = [&](int g) -> v4u {
-        const int t = 16 * g + tl;
-        return ds128v(b.x + (t * 16 + (pb ^ (t & 15))) * 16);
-    };
-    const v4u z = {0u, 0u, 0u, 0u};
-    f.b0 = bfrag(0);
-    f.b1 = G > 1 ? bfrag(1) : z;
-    f.b2 = G > 2 ? bfrag(2) : z;
-    f.b3 = G > 3 ? bfrag(3) : z;
-    return f;
-}
-__device__ __forceinline__ void kq_f64_wait(KqF64& f) {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f.a), "+v"(f.b0), "+v"(f.b1), "+v"(f.b2), "+v"(f.b3));
 }
 
 // Each byte of q (0..15) times d (0..7), as two 16-bit lanes a dword (v_pk_mul_lo_u16, full rate,
@@ -586,67 +534,6 @@ __device__ __forceinline__ uint32_t mul_bytes1(uint32_t q, u16x2 dd) {
 __device__ __forceinline__ v4u mul_bytes(const v4u& q, uint32_t d) {
     const u16x2 dd = {static_cast<unsigned short>(d), static_cast<unsigned short>(d)};
     return v4u{mul_bytes1(q.x, dd), mul_bytes1(q.y, dd), mul_bytes1(q.z, dd), mul_bytes1(q.w, dd)};
-}
-
-template <int G>
-__device__ __forceinline__ void kq_compute_fold(const KqBases& base, MmAcc<G>& acc) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tl = lane & 15, l16 = lane >> 4;
-    const int ar = wave * 16 + tl, orow0 = wave * 16 + l16 * 4;
-    const v4i zero = {0, 0, 0, 0};
-    // the A row's decoded scales and mins (for the digits), the output rows' d / dmin, the groups' x scales
-    v4u scm = ds128v(base.wk + 1024 + ar * 16);
-    uint32_t dd[4], xd[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        dd[i] = ds32(base.wk + (orow0 + i) * 16);
-        xd[i] = i < G ? ds32(base.xd + (16 * i + tl) * 4) : 0u;
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(scm), "+v"(dd[0]), "+v"(dd[1]), "+v"(dd[2]), "+v"(dd[3]), "+v"(xd[0]), "+v"(xd[1]), "+v"(xd[2]),
-                   "+v"(xd[3]));
-    KqF64 cur = kq_f64_issue<G>(base, 0, ar, tl, l16);
-    kq_f64_wait(cur);
-    v4i alo[4], ahi[4], amn[4];
-#pragma unroll
-    for (int g = 0; g < G; ++g) alo[g] = ahi[g] = amn[g] = zero;
-    // lanes 32..63 take the odd sub-block of the pair (high nibbles): a shift by 4, not a select
-    const uint32_t nib_shift = l16 >= 2 ? 4u : 0u;
-    const uint32_t lane_byte = static_cast<uint32_t>(l16 >> 1) * 0x01010101u;
-#pragma unroll
-    for (int st = 0; st < 4; ++st) {
-        KqF64 nxt;
-        if (st < 3) nxt = kq_f64_issue<G>(base, st + 1, ar, tl, l16);
-        const int j = 2 * st + (l16 >> 1);  // this lane's sub-block (j < 4 exactly when st < 2)
-        const uint32_t sc = ((st < 2 ? scm.x : scm.y) >> (8 * (j & 3))) & 0xFF;
-        // the min byte of sub-block j in all four bytes (v_perm_b32: byte j & 3 of the word, four times)
-        const uint32_t m4 = __builtin_amdgcn_perm(0u, st < 2 ? scm.z : scm.w, lane_byte + static_cast<uint32_t>((2 * st) & 3) * 0x01010101u);
-        const uint32_t dlo = sc & 7, dhi = sc >> 3;
-        const v4u qn = (cur.a >> nib_shift) & 0x0F0F0F0Fu;
-        const v4u qlo = mul_bytes(qn, dlo);  // bytes 0..15 times 0..7: no carries between bytes
-        const v4u qhi = mul_bytes(qn, dhi);
-        const v4u qmn = {m4, m4, m4, m4};
-        const v4u bq[4] = {cur.b0, cur.b1, cur.b2, cur.b3};
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            alo[g] = mfma64(qlo, bq[g], alo[g]);
-            ahi[g] = mfma64(qhi, bq[g], ahi[g]);
-            amn[g] = mfma64(qmn, bq[g], amn[g]);
-        }
-        if (st < 3) {
-            kq_f64_wait(nxt);
-            cur = nxt;
-        }
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const float xg = __uint_as_float(xd[g]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int weighted = alo[g][i] + 8 * ahi[g][i], offsets = amn[g][i];
-            const float d = h2f(static_cast<uint16_t>(dd[i] & 0xFFFF)), dmin = h2f(static_cast<uint16_t>(dd[i] >> 16));
-            acc.s[g][i] += xg * (d * static_cast<float>(weighted) - dmin * static_cast<float>(offsets));  // src/quant.cpp:500-521
-        }
-    }
 }
 
 // Q6_K with its signed 8-bit scales folded into the MFMAs.  Per 16-value
@@ -673,12 +560,12 @@ __device__ __forceinline__ Kq6F kq6_issue(uint32_t base, int st, int ar, int tl,
     Kq6F f;
     const int half = st >> 1;
     const int lp = half * 4 + l16, hp = half * 2 + (l16 & 1);
-    f.l = ds128v(base + offsetof(KqStage<kQ6_K>, w0) + (ar * 8 + (lp ^ (ar & 7))) * 16);
-    f.h = ds128v(base + offsetof(KqStage<kQ6_K>, wk) + (ar * 4 + (hp ^ (ar & 3))) * 16);
+    f.l = ds128v(base + offsetof(KqStage, w0) + (ar * 8 + (lp ^ (ar & 7))) * 16);
+    f.h = ds128v(base + offsetof(KqStage, wk) + (ar * 4 + (hp ^ (ar & 3))) * 16);
     const int pb = 4 * st + l16;
     auto bfrag = [&](int g) -> v4u {
         const int t = 16 * g + tl;
-        return ds128v(base + offsetof(KqStage<kQ6_K>, x) + (t * 16 + (pb ^ (t & 15))) * 16);
+        return ds128v(base + offsetof(KqStage, x) + (t * 16 + (pb ^ (t & 15))) * 16);
     };
     const v4u z = {0u, 0u, 0u, 0u};
     f.b0 = bfrag(0);
@@ -697,13 +584,13 @@ __device__ __forceinline__ void kq_compute_fold6(uint32_t base, MmAcc<G>& acc) {
     const int ar = wave * 16 + tl, orow0 = wave * 16 + l16 * 4;
     const v4i zero = {0, 0, 0, 0};
     // the A row's 16 int8 scales (four dwords of its meta), the output rows' d, the groups' x scales
-    const uint32_t arow = base + offsetof(KqStage<kQ6_K>, wm) + ar * 20;
+    const uint32_t arow = base + offsetof(KqStage, wm) + ar * 20;
     uint32_t s0 = ds32(arow), s1 = ds32(arow + 4), s2 = ds32(arow + 8), s3 = ds32(arow + 12);
     uint32_t dd[4], xd[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        dd[i] = ds32(base + offsetof(KqStage<kQ6_K>, wm) + (orow0 + i) * 20 + 16);
-        xd[i] = i < G ? ds32(base + offsetof(KqStage<kQ6_K>, xd) + (16 * i + tl) * 4) : 0u;
+        dd[i] = ds32(base + offsetof(KqStage, wm) + (orow0 + i) * 20 + 16);
+        xd[i] = i < G ? ds32(base + offsetof(KqStage, xd) + (16 * i + tl) * 4) : 0u;
     }
     asm volatile("s_waitcnt lgkmcnt(0)"
                  : "+v"(s0), "+v"(s1), "+v"(s2), "+v"(s3), "+v"(dd[0]), "+v"(dd[1]), "+v"(dd[2]), "+v"(dd[3]), "+v"(xd[0]),
@@ -1066,7 +953,7 @@ __global__ __launch_bounds__(64 * W) void k_mmx(MmArgs g) {
     }
 }
 
-// ---------------------------------------------------------------- the GEMM of the 32-value formats and TQ2_0
+// ---------------------------------------------------------------- the GEMM of the 32-value formats, TQ2_0 and Q4_K
 
 // Tokens are the MFMA's rows (A), weight rows its columns (B): v_mfma_i32_32x32x32_i8 takes one 32-value
 // block a step (K = 32), and D holds, in lane l, weight row l % 32 and tokens 8 (i / 4) + 4 (l / 32) + i % 4.
@@ -1083,10 +970,15 @@ __global__ __launch_bounds__(64 * W) void k_mmx(MmArgs g) {
 // 4- and 5-bit values enter scaled by 16 or 8, which puts them at the top of the int8 with a shift and an
 // xor; d_w takes the factor back, exactly.
 //
+// The pair's waves are half gate rows and half up rows of the same 64, traded through LDS at the end: with both
+// matrices in every wave the registers held one workgroup a compute unit (Q8_0 pair of 6144 x 2048, 512 tokens:
+// 113 us, now 75; Q4_K pair of 8192 x 2048: 84, now 66).
+//
 // Q8_0 6144 x 2048, 512 tokens: 44 us, 0.29 Pop/s (the form before, 16 x 16 MFMAs with a conversion and three
 // scale reads an output, 82 us).  55% of the vector unit's issue slots are full: 187 registers hold two
-// workgroups a compute unit, whose 768 tiles are one and a half rounds.  A few tokens are bound by the chunk's
-// latency instead (1.7 us a chunk and workgroup).
+// workgroups a compute unit, whose 768 tiles are one and a half rounds.  Q4_K 8192 x 2048 pair, 512 tokens:
+// 66 us (70 before, as a 64-row kernel that staged both matrices).  Reading further ahead (two or three chunks)
+// gave nothing at any tile: what a chunk takes is its instructions.
 constexpr int kMgWaves = 4;
 
 // Store, add, or gate/up pair of up to kMgMats matrices of one format over the same rows of activations.
@@ -1097,6 +989,8 @@ struct MgArgs {
     float* out[kMgMats];
     int ostride[kMgMats];
     int tiles[kMgMats];  // workgroup row tiles of each
+    const int8_t* qx[kMgMats];   // Q6_K: the expanded planes
+    const float* qxd[kMgMats];
 };
 
 constexpr float kMgMagic = 12582912.0f;  // 1.5 * 2^23
@@ -1122,6 +1016,7 @@ template <uint32_t T>
 struct MgWave {
     v4u q[32 * mg_pieces<T>()];
     uint4 e[T == kTQ2_0 ? 1 : 64];   // row r's 8 fp16 scales at r; Q4_1: its offsets at 32 + r
+                                     // Q4_K: its decoded scales and mins at r, {d, dmin} at 32 + r
     uint4 f[T == kQ5_0 ? 64 : 1];    // Q5_0: row r's 8 words of fifth bits at 2 r, 2 r + 1
     float d[T == kTQ2_0 ? 32 : 1];   // TQ2_0: row r's scale
 };
@@ -1131,18 +1026,20 @@ template <uint32_t T>
 __device__ __forceinline__ void mg_load(MgRegs<T>& w, const Packed& m, uint32_t r0, int c, int nb) {
     constexpr int P = mg_pieces<T>();
     const int lane = threadIdx.x & 63;
-    const uint32_t rmax = m.rows - 1, units = T == kTQ2_0 ? m.cols / 256 : m.cols / 32;
-    const int last = T == kQ8_0 ? 2 * nb - 1 : T == kTQ2_0 ? 3 : nb - 1;
+    const uint32_t rmax = m.rows - 1, units = T == kTQ2_0 || T == kQ4_K ? m.cols / 256 : m.cols / 32;
+    const int last = T == kQ8_0 ? 2 * nb - 1 : T == kTQ2_0 ? 3 : T == kQ4_K ? 7 : nb - 1;
     auto row_of = [&](int r) -> size_t { return r0 + r <= rmax ? r0 + r : rmax; };
 #pragma unroll
     for (int k = 0; k < P / 2; ++k) {
         const int i = k * 64 + lane, r = i / P, p = i % P < last ? i % P : last;
         const size_t blk = row_of(r) * units;
-        const uint8_t* base = T == kTQ2_0 ? m.p0 + (blk + c) * 64 : m.p0 + (blk + 8 * c) * (T == kQ8_0 ? 32 : 16);
+        const uint8_t* base = T == kTQ2_0 ? m.p0 + (blk + c) * 64 : T == kQ4_K ? m.p0 + (blk + c) * 128 : m.p0 + (blk + 8 * c) * (T == kQ8_0 ? 32 : 16);
         w.q[k] = *gmem(reinterpret_cast<const v4u*>(base) + p);
     }
     if constexpr (T == kTQ2_0) {
         w.e.x = gld<uint16_t>(m.p1, row_of(lane & 31) * units + c);
+    } else if constexpr (T == kQ4_K) {
+        w.e = ld16((lane < 32 ? m.p2 : m.p1) + (row_of(lane & 31) * units + c) * 16);
     } else {
         if (lane < 32 || T == kQ4_1) w.e = chunk_halves(lane < 32 ? m.p1 : m.p2, row_of(lane & 31) * units + 8 * c, nb);
         if constexpr (T == kQ5_0) {
@@ -1170,7 +1067,7 @@ __device__ __forceinline__ void mg_put(MgWave<T>& L, const MgRegs<T>& w) {
     if constexpr (T == kTQ2_0) {
         if (lane < 32) L.d[lane] = h2f(static_cast<uint16_t>(w.e.x));
     } else {
-        if (lane < 32 || T == kQ4_1) L.e[lane] = w.e;
+        if (lane < 32 || T == kQ4_1 || T == kQ4_K) L.e[lane] = w.e;
         if constexpr (T == kQ5_0) L.f[lane] = w.f;
     }
 }
@@ -1184,7 +1081,7 @@ __device__ __forceinline__ MgS mg_scales(const MgWave<T>& L) {
     const int r = threadIdx.x & 31;
     MgS s{};
     if constexpr (T != kTQ2_0) s.sc = L.e[r];
-    if constexpr (T == kQ4_1) s.mn = L.e[32 + r];
+    if constexpr (T == kQ4_1 || T == kQ4_K) s.mn = L.e[32 + r];
     if constexpr (T == kQ5_0) {
         s.qh[0] = L.f[2 * r];
         s.qh[1] = L.f[2 * r + 1];
@@ -1235,81 +1132,120 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
-template <uint32_t T, int TG, int NM>
+// Q4_K: a super-block's values with the scales folded in, for sub-block j sc = lo + 8 hi (3-bit digits: q lo and q hi fit int8),
+//   weighted = sum_j sc_j dot_j = A_lo + 8 A_hi,  A_lo = sum_k (q_k lo_j(k)) x_k,
+// two exact int32 chains of 8 MFMAs (dot_q4_k_q8_k, src/quant.cpp:500-521).  The offsets sum_j mn_j pair_j are one fp16 MFMA of the mins (0 .. 63,
+// each twice) and the sums of 16 activations (at most 2048: exact in fp16); its float sums stay below 2^24,
+// so they are the integer exactly.
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ v4u mg_mins(uint32_t m4) {
+    v4u r;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float f = static_cast<float>((m4 >> (8 * k)) & 0xFF);
+        r[k] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(f, f));
+    }
+    return r;
+}
+
+// The gated output (a table is filled first: exp_tab_fill).
+__device__ __forceinline__ float mg_gate(const MmArgs& g, float gv, float up) {
+    if (g.relu2) {
+        const float q = gv > 0.0f ? gv : 0.0f;
+        return q * q * up;  // src/model.cpp:1134-1138
+    }
+    if (g.gelu) return gelu_mul(gv, up);  // src/kernels_f32.cpp:291-296
+    return gv / (1.0f + ref_expf_s(-gv)) * up;  // src/kernels_f32.cpp:287-289
+}
+// Row groups of 32 a workgroup: the pair's waves are half gate, half up.
+template <int MODE>
+__host__ __device__ constexpr int mg_row_waves() { return MODE == kMmPair ? kMgWaves / 2 : kMgWaves; }
+
+template <uint32_t T, int TG>
 struct MgLds {
     alignas(16) int8_t b[2][8 * TG][kBRow];
-    alignas(16) float xd[2][T == kTQ2_0 ? 1 : 8][8 * TG];   // [block][token]
+    alignas(16) uint32_t bs[2][T == kQ4_K ? 8 * TG : 1][8 + 4];  // Q4_K: the 16 sums as fp16
+    alignas(16) float xd[2][T == kTQ2_0 || T == kQ4_K ? 1 : 8][8 * TG];   // [block][token]
     alignas(16) float xs[2][T == kQ4_1 ? 8 : 1][8 * TG];    // Q4_1: d_x * sum
-    alignas(16) MgWave<T> w[kMgWaves][NM];
+    alignas(16) MgWave<T> w[kMgWaves];
 };
 
 template <uint32_t T, int MODE, int TG>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_mg(MgArgs ga) {
-    constexpr int kTok = 8 * TG, NM = MODE == kMmPair ? 2 : 1;
-    __shared__ MgLds<T, TG, NM> L;
-    constexpr bool kSums = T == kQ4_1, q8k = T == kTQ2_0;
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, TG == 4 ? 4 : 2))) void k_mg(MgArgs ga) {
+    constexpr int kTok = 8 * TG, kRowWaves = mg_row_waves<MODE>();
+    __shared__ MgLds<T, TG> L;
+    constexpr bool kSums = T == kQ4_1, q8k = T == kTQ2_0 || T == kQ4_K;
     const MmArgs& g = ga.a;
     int tile = blockIdx.x, ti = 0;
     while (ti < kMgMats - 1 && tile >= ga.tiles[ti]) tile -= ga.tiles[ti++];
-    const Packed m = ga.m[ti];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5;
-    const uint32_t r0 = (static_cast<uint32_t>(tile) * kMgWaves + wave) * 32, rmax = m.rows - 1;
+    const Packed m = MODE == kMmPair && wave >= kRowWaves ? g.m2 : ga.m[ti];
+    const uint32_t r0 = (static_cast<uint32_t>(tile) * kRowWaves + wave % kRowWaves) * 32, rmax = m.rows - 1;
     const uint32_t row = r0 + (lane & 31) <= rmax ? r0 + (lane & 31) : rmax;
     const int t0 = blockIdx.y * kTok;
     const bool lut16 = (m.flags & kFlagLut16) != 0;
     const int nc = static_cast<int>((m.cols + kChunkCols - 1) / kChunkCols), nsub = static_cast<int>(m.cols / 32);
     auto nb_of = [&](int c) { return nsub - 8 * c < 8 ? nsub - 8 * c : 8; };
 
-    // the workgroup's activations of a chunk, through registers: pieces of 16 bytes, and the scales
+    // the workgroup's activations of a chunk, through registers: pieces of 16 bytes, the scales and sums
     constexpr int kPieces = (kTok * 16 + kThreads - 1) / kThreads;
-    uint4 aq[kPieces];
-    float ad = 0.0f, as = 0.0f;
+    struct Act {
+        uint4 q[kPieces];
+        float d, s;
+        uint64_t b;  // Q4_K: two sums
+    };
     auto tokc = [&](int t) -> size_t { return static_cast<size_t>(t0 + t < g.ntok ? t0 + t : g.ntok - 1); };
-    auto act_load = [&](int c) {
+    auto act_load = [&](Act& x, int c) {
 #pragma unroll
         for (int k = 0; k < kPieces; ++k) {
             const int i = k * kThreads + tid;
-            if (kTok * 16 % kThreads == 0 || i < kTok * 16) aq[k] = ld16(reinterpret_cast<const uint8_t*>(g.x.qs) + tokc(i >> 4) * g.x.stride + c * kChunkCols + (i & 15) * 16);
+            if (kTok * 16 % kThreads == 0 || i < kTok * 16) x.q[k] = ld16(reinterpret_cast<const uint8_t*>(g.x.qs) + tokc(i >> 4) * g.x.stride + c * kChunkCols + (i & 15) * 16);
         }
         if (q8k) {
-            if (tid < kTok) ad = gld<float>(g.x.d, tokc(tid) * (g.x.stride / 32) + c);
+            if (tid < kTok) x.d = gld<float>(g.x.d, tokc(tid) * (g.x.stride / 32) + c);
+            if (T == kQ4_K && tid < kTok * 8) x.b = gld<uint64_t>(g.x.bs, (tokc(tid >> 3) * (g.x.stride / 16) + c * 16) / 2 + (tid & 7));
         } else if (tid < kTok * 8) {
-            ad = gld<float>(g.x.d, tokc(tid >> 3) * (g.x.stride / 32) + c * 8 + (tid & 7));
-            if (kSums) as = ad * static_cast<float>(gld<int32_t>(g.x.bs, tokc(tid >> 3) * (g.x.stride / 16) + c * 8 + (tid & 7)));
+            x.d = gld<float>(g.x.d, tokc(tid >> 3) * (g.x.stride / 32) + c * 8 + (tid & 7));
+            if (kSums) x.s = x.d * static_cast<float>(gld<int32_t>(g.x.bs, tokc(tid >> 3) * (g.x.stride / 16) + c * 8 + (tid & 7)));
         }
     };
-    auto act_store = [&](int s) {
+    auto act_store = [&](const Act& x, int s) {
 #pragma unroll
         for (int k = 0; k < kPieces; ++k) {
             const int i = k * kThreads + tid;
-            if (kTok * 16 % kThreads == 0 || i < kTok * 16) *reinterpret_cast<uint4*>(&L.b[s][i >> 4][(i & 15) * 16]) = aq[k];
+            if (kTok * 16 % kThreads == 0 || i < kTok * 16) *reinterpret_cast<uint4*>(&L.b[s][i >> 4][(i & 15) * 16]) = x.q[k];
         }
         if (q8k) {
-            if (tid < kTok) L.xd[s][0][tid] = ad;
+            if (tid < kTok) L.xd[s][0][tid] = x.d;
+            if (T == kQ4_K && tid < kTok * 8)
+                L.bs[s][tid >> 3][tid & 7] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(static_cast<float>(static_cast<int32_t>(x.b)), static_cast<float>(static_cast<int32_t>(x.b >> 32))));
         } else if (tid < kTok * 8) {
-            L.xd[s][tid & 7][tid >> 3] = ad;
-            if (kSums) L.xs[s][tid & 7][tid >> 3] = as;
+            L.xd[s][tid & 7][tid >> 3] = x.d;
+            if (kSums) L.xs[s][tid & 7][tid >> 3] = x.s;
         }
     };
 
-    if (MODE == kMmPair) exp_tab_fill();  // ordered before the epilogue by the loop's barriers
-    MgRegs<T> w[NM];
-    const Packed mm[2] = {m, NM == 2 ? g.m2 : m};
-    act_load(0);
-#pragma unroll
-    for (int n = 0; n < NM; ++n) mg_load<T>(w[n], mm[n], r0, 0, nb_of(0));
-#pragma unroll
-    for (int n = 0; n < NM; ++n) mg_put<T>(L.w[wave][n], w[n]);
-    act_store(0);
+    if (MODE == kMmPair || MODE == kMmGated) exp_tab_fill();  // ordered before the epilogue by the loop's barriers
+    MgRegs<T> w;  // the next chunk's
+    Act act;
+    auto load = [&](int c) {
+        act_load(act, c);
+        mg_load<T>(w, m, r0, c, nb_of(c));
+    };
+    auto put = [&](int c) {
+        mg_put<T>(L.w[wave], w);
+        act_store(act, c & 1);
+    };
+    load(0);
+    put(0);
     __syncthreads();
-    float acc[NM][4 * TG];
+    float acc[4 * TG];
 #pragma unroll
-    for (int n = 0; n < NM; ++n)
-#pragma unroll
-        for (int i = 0; i < 4 * TG; ++i) acc[n][i] = 0.0f;
+    for (int i = 0; i < 4 * TG; ++i) acc[i] = 0.0f;
     v16i magic;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) magic[i] = q8k ? 0 : 0x4B400000;
+    for (int i = 0; i < 16; ++i) magic[i] = 0x4B400000;
     if (!q8k) asm volatile("" : "+v"(magic));  // held in registers, not rebuilt for every MFMA
     const int atok = (lane & 31) & (kTok - 1);  // A's row (rows past the tile's tokens: copies, never read)
     // the token of this lane's half's output i = l % 16: a 16-lane row holds its half's token scales, one
@@ -1319,82 +1255,96 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
 
     for (int c = 0; c < nc; ++c) {
         const int s = c & 1, nb = nb_of(c);
-        if (c + 1 < nc) {
-            act_load(c + 1);
-#pragma unroll
-            for (int n = 0; n < NM; ++n) mg_load<T>(w[n], mm[n], r0, c + 1, nb_of(c + 1));
-        }
-        MgS sc[NM];
-#pragma unroll
-        for (int n = 0; n < NM; ++n) sc[n] = mg_scales<T>(L.w[wave][n]);
+        const MgWave<T>& W = L.w[wave];
+        if (c + 1 < nc) load(c + 1);
+        const MgS sc = mg_scales<T>(W);
         auto afrag = [&](int jj) { return *reinterpret_cast<const v4u*>(&L.b[s][atok][jj * 32 + 16 * h]); };
-        if constexpr (T == kTQ2_0) {
-            v16i d[NM];
-#pragma unroll
-            for (int n = 0; n < NM; ++n) d[n] = magic;
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {  // the block's int32 sum over its 8 steps, exact
-                const v4u a = afrag(jj);
-#pragma unroll
-                for (int n = 0; n < NM; ++n) d[n] = mfma32(a, mg_frag<T>(L.w[wave][n], sc[n], jj, h), d[n]);
-            }
-            float wd[NM];
-#pragma unroll
-            for (int n = 0; n < NM; ++n) wd[n] = L.w[wave][n].d[lane & 31];
+        if constexpr (T == kQ4_K) {
+            const v8h sums = *reinterpret_cast<const v8h*>(&L.bs[s][atok][4 * h]);
             const float xv = L.xd[s][0][stok];
+            v16i lo = {}, hi = {};
+#pragma unroll
+            for (int jp = 0; jp < 4; ++jp) {
+                const int r = lane & 31;
+                const v4u q = W.q[r * 8 + ((2 * jp + h) ^ mg_swz<T>(r))];
+#pragma unroll
+                for (int o = 0; o < 2; ++o) {
+                    const int jj = 2 * jp + o;
+                    const v4u a = afrag(jj), qn = (q >> (4u * o)) & 0x0F0F0F0Fu;
+                    const uint32_t sb = u4_word(sc.sc, jj >> 2) >> (8 * (jj & 3));
+                    lo = mfma32(a, mul_bytes(qn, sb & 7), lo);
+                    hi = mfma32(a, mul_bytes(qn, (sb >> 3) & 7), hi);
+                }
+            }
+            const v16f off = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, __builtin_bit_cast(v8h, mg_mins(h ? sc.sc.w : sc.sc.z)), v16f{}, 0, 0, 0);
+            const float dw = h2f(static_cast<uint16_t>(sc.mn.x & 0xFFFF)), dmin = h2f(static_cast<uint16_t>(sc.mn.x >> 16));
             static_for<4 * TG>([&](auto ic) {
                 constexpr int i = decltype(ic)::value;
-                const float xd = row_bcast<i>(xv);
+                const int weighted = lo[i] + 8 * hi[i];
+                acc[i] += row_bcast<i>(xv) * (dw * static_cast<float>(weighted) - dmin * off[i]);  // src/quant.cpp:500-521
+            });
+        } else if constexpr (T == kTQ2_0) {
+            v16i d = {};
 #pragma unroll
-                for (int n = 0; n < NM; ++n) {
-                    const float v = static_cast<float>(d[n][i]);
-                    acc[n][i] += lut16 ? v * wd[n] * xd : xd * wd[n] * v;  // src/quant.cpp:789-802 / :580-596
-                }
+            for (int jj = 0; jj < 8; ++jj) d = mfma32(afrag(jj), mg_frag<T>(W, sc, jj, h), d);  // the block's int32 sum, exact
+            const float wd = W.d[lane & 31], xv = L.xd[s][0][stok];
+            static_for<4 * TG>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const float xd = row_bcast<i>(xv), v = static_cast<float>(d[i]);
+                acc[i] += lut16 ? v * wd * xd : xd * wd * v;  // src/quant.cpp:789-802 / :580-596
             });
         } else {
-            bool odd = nb < 8;
-#pragma unroll
-            for (int n = 0; n < NM; ++n) odd = odd || halves_not_finite(sc[n].sc);
-            auto dots = [&](int jj, int n) { return mfma32(afrag(jj), mg_frag<T>(L.w[wave][n], sc[n], jj, h), magic); };
+            const bool odd = nb < 8 || halves_not_finite(sc.sc);
+            auto dots = [&](int jj) { return mfma32(afrag(jj), mg_frag<T>(W, sc, jj, h), magic); };
             auto half_at = [](const uint4& v, int jj) {
                 const uint32_t word = u4_word(v, jj >> 1);
                 return h2f(static_cast<uint16_t>((jj & 1) ? (word >> 16) : (word & 0xFFFF)));
             };
-            auto terms = [&](auto fast, int jj, int n, const v16i& d) {
-                const float wd = half_at(sc[n].sc, jj) * mg_unscale<T>(), cw = -kMgMagic * wd;
-                const float wm = kSums ? half_at(sc[n].mn, jj) : 0.0f;
+            auto terms = [&](auto fast, int jj, const v16i& d) {
+                const float wd = half_at(sc.sc, jj) * mg_unscale<T>(), cw = -kMgMagic * wd;
+                const float wm = kSums ? half_at(sc.mn, jj) : 0.0f;
                 const float xv = L.xd[s][jj][stok], sv = kSums ? L.xs[s][jj][stok] : 0.0f;
                 static_for<4 * TG>([&](auto ic) {
                     constexpr int i = decltype(ic)::value;
                     const float f = __int_as_float(d[i]);
                     const float p = decltype(fast)::value ? __builtin_fmaf(f, wd, cw) : (f - kMgMagic) * wd;
-                    if constexpr (kSums) acc[n][i] += row_bcast<i>(xv) * p + row_bcast<i>(sv) * wm;
-                    else acc[n][i] += row_bcast<i>(xv) * p;
+                    if constexpr (kSums) acc[i] += row_bcast<i>(xv) * p + row_bcast<i>(sv) * wm;
+                    else acc[i] += row_bcast<i>(xv) * p;
                 });
             };
             if (__builtin_amdgcn_ballot_w64(odd) == 0) {  // the next dots under these terms
                 v16i d[2];
-                d[0] = dots(0, 0);
+                d[0] = dots(0);
 #pragma unroll
-                for (int u = 0; u < 8 * NM; ++u) {
-                    if (u + 1 < 8 * NM) d[(u + 1) & 1] = dots((u + 1) / NM, (u + 1) % NM);
-                    terms(std::true_type{}, u / NM, u % NM, d[u & 1]);
+                for (int jj = 0; jj < 8; ++jj) {
+                    if (jj + 1 < 8) d[(jj + 1) & 1] = dots(jj + 1);
+                    terms(std::true_type{}, jj, d[jj & 1]);
                 }
             } else {  // the row ends inside the chunk, or a scale is not finite
 #pragma unroll
                 for (int jj = 0; jj < 8; ++jj) {
                     if (jj >= nb) break;  // past the row: no term
-#pragma unroll
-                    for (int n = 0; n < NM; ++n) terms(std::false_type{}, jj, n, dots(jj, n));
+                    terms(std::false_type{}, jj, dots(jj));
                 }
             }
         }
-        if (c + 1 < nc) {
-            act_store(s ^ 1);
-#pragma unroll
-            for (int n = 0; n < NM; ++n) mg_put<T>(L.w[wave][n], w[n]);
-        }
+        if (c + 1 < nc) put(c + 1);
         __syncthreads();
+    }
+    if constexpr (MODE == kMmPair) {  // a gate wave and its up wave take half of their outputs each, through LDS
+        float(*x)[4 * TG][64] = reinterpret_cast<float(*)[4 * TG][64]>(&L.b[0][0][0]);
+        static_assert(sizeof(L.b) >= kMgWaves * 4 * TG * 64 * sizeof(float));
+#pragma unroll
+        for (int i = 0; i < 4 * TG; ++i) x[wave][i][lane] = acc[i];
+        __syncthreads();
+        if (r0 + (lane & 31) > rmax) return;
+        const int gw = wave % kRowWaves, o0 = wave >= kRowWaves ? 2 * TG : 0;
+#pragma unroll 1
+        for (int o = o0; o < o0 + 2 * TG; ++o) {  // one copy of the gates' code: unrolled, its 28 KB were fetched for 8 outputs
+            const int t = t0 + 8 * (o >> 2) + 4 * h + (o & 3);
+            if (t < g.ntok) ga.out[ti][static_cast<size_t>(t) * ga.ostride[ti] + row] = mg_gate(g, x[gw][o][lane], x[gw + kRowWaves][o][lane]);
+        }
+        return;
     }
     if (r0 + (lane & 31) > rmax) return;
 #pragma unroll
@@ -1402,40 +1352,232 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 4))
         const int t = t0 + 8 * (i >> 2) + 4 * h + (i & 3);
         if (t >= g.ntok) continue;
         float* o = ga.out[ti] + static_cast<size_t>(t) * ga.ostride[ti] + row;
-        const float v = acc[0][i];
-        if (MODE == kMmStore) {
-            *o = v;
-        } else if (MODE == kMmAdd) {
-            *o = *o + v;  // h += proj (src/model.cpp:1111, :1162)
+        if (MODE == kMmStore) *o = acc[i];
+        else if (MODE == kMmAdd) *o = *o + acc[i];  // h += proj (src/model.cpp:1111, :1162)
+        else *o = mg_gate(g, *o, acc[i]);          // kMmGated: out holds the gate row, this is up
+    }
+}
+
+// ---------------------------------------------------------------- the same, K split over a workgroup's waves
+
+// With few tokens and rows a launch of k_mg has few waves, and each is a chain: a chunk is some 350
+// instructions of one wave, about 1 us, whatever is read ahead.  Here a workgroup computes 32 rows x 8
+// tokens and its waves share the chunks: wave w forms the terms of chunks w, w + W, ... in registers and,
+// when the chunk before has been added, adds its own in block order (the sums stay the reference's bit for
+// bit) and passes the accumulators on through LDS.  Only the adds are serial.  Wave w waits for wave w - 1 of
+// the same workgroup, whose waves are all resident.  Q6_K multiplies its expanded planes.
+constexpr int kMgsWaves = 8;
+constexpr int kMgsTok = 8;
+template <int MODE>
+__host__ __device__ constexpr int mgs_split() { return MODE == kMmPair ? kMgsWaves / 2 : kMgsWaves; }  // waves a matrix
+
+template <uint32_t T>
+__host__ __device__ constexpr bool mgs_q8k() { return T == kTQ2_0 || T == kQ4_K || T == kQ6_K; }
+
+template <uint32_t T>
+struct MgsIn {  // a wave's operands of a chunk, in flight
+    MgRegs<T> w;
+    v4u a[8];
+    float d[mgs_q8k<T>() ? 1 : 8];
+    int32_t bs[T == kQ4_1 || T == kQ4_K ? 8 : 1];
+};
+template <>
+struct MgsIn<kQ6_K> {
+    v4u lo[8], hi[8], a[8];
+    float wd, d[1];
+};
+
+template <uint32_t T, int MODE>
+__global__ __launch_bounds__(64 * kMgsWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_mgs(MgArgs ga) {
+    constexpr int W = mgs_split<MODE>(), kMats = kMgsWaves / W;
+    constexpr bool kSums = T == kQ4_1, q8k = mgs_q8k<T>(), kSplitQ6 = T == kQ6_K;
+    constexpr int kTerms = q8k ? 1 : 8;  // terms a chunk and output
+    __shared__ MgWave<kSplitQ6 ? kTQ2_0 : T> wl[kSplitQ6 ? 1 : kMgsWaves];
+    __shared__ float accl[kMats][4][64];
+    __shared__ int turn[kMats];  // chunks added
+    const MmArgs& g = ga.a;
+    int tile = blockIdx.x, ti = 0;
+    while (ti < kMgMats - 1 && tile >= ga.tiles[ti]) tile -= ga.tiles[ti++];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5, mat = wave / W, kw = wave % W;
+    const Packed m = MODE == kMmPair && mat == 1 ? g.m2 : ga.m[ti];
+    const uint32_t r0 = static_cast<uint32_t>(tile) * 32, rmax = m.rows - 1;
+    const uint32_t row = r0 + (lane & 31) <= rmax ? r0 + (lane & 31) : rmax;
+    const int t0 = blockIdx.y * kMgsTok;
+    const bool lut16 = (m.flags & kFlagLut16) != 0;
+    const int nc = static_cast<int>((m.cols + kChunkCols - 1) / kChunkCols), nsub = static_cast<int>(m.cols / 32);
+    auto nb_of = [&](int c) { return nsub - 8 * c < 8 ? nsub - 8 * c : 8; };
+    auto tokc = [&](int t) -> size_t { return static_cast<size_t>(t0 + t < g.ntok ? t0 + t : g.ntok - 1); };
+    const size_t ta = tokc(lane & 7), ts = tokc(4 * h + (lane & 3));  // A's row (8 tokens, four times) and the outputs' token scales
+    const uint8_t* xq = reinterpret_cast<const uint8_t*>(g.x.qs) + ta * g.x.stride + 16 * h;
+    const float* xd = g.x.d + ts * (g.x.stride / 32);
+    if (tid < kMats) turn[tid] = 0;
+    if (MODE == kMmPair) exp_tab_fill();
+    __syncthreads();
+
+    auto load = [&](MgsIn<T>& in, int c) {
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) in.a[jj] = *gmem(reinterpret_cast<const v4u*>(xq + c * kChunkCols + jj * 32));
+        if constexpr (q8k) {
+            in.d[0] = gld<float>(xd, c);
         } else {
-            const float up = acc[NM - 1][i];
-            if (g.relu2) {
-                const float q = v > 0.0f ? v : 0.0f;
-                *o = q * q * up;  // src/model.cpp:1134-1138
-            } else if (g.gelu) {
-                *o = gelu_mul(v, up);  // src/kernels_f32.cpp:291-296
+#pragma unroll
+            for (int k = 0; k < 8; ++k) in.d[k] = gld<float>(xd, c * 8 + k);
+        }
+        if constexpr (T == kQ4_1) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) in.bs[k] = gld<int32_t>(g.x.bs, ts * (g.x.stride / 16) + c * 8 + k);
+        }
+        if constexpr (T == kQ4_K) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) in.bs[k] = gld<int32_t>(g.x.bs, ta * (g.x.stride / 16) + c * 16 + 8 * h + k);
+        }
+        if constexpr (kSplitQ6) {
+            const size_t rc = static_cast<size_t>(r0 / 32) * nc + c;
+            const int8_t* qx = ga.qx[ti];
+            const auto* f = gmem(reinterpret_cast<const v4u*>(qx + rc * 16384)) + lane;
+#pragma unroll
+            for (int jj = 0; jj < 8; ++jj) {
+                in.lo[jj] = f[2 * jj * 64];
+                in.hi[jj] = f[(2 * jj + 1) * 64];
+            }
+            in.wd = gld<float>(ga.qxd[ti], rc * 32 + (lane & 31));
+        } else {
+            mg_load<T>(in.w, m, r0, c, nb_of(c));
+        }
+    };
+
+    float acc[4] = {};
+    MgsIn<T> in;
+    if (kw < nc) load(in, kw);
+    for (int c = kw; c < nc; c += W) {
+        const int nb = nb_of(c), next = c + W;
+        float p[kTerms][4];
+        v4u a[8];
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) a[jj] = in.a[jj];
+        if constexpr (kSplitQ6) {
+            v16i lo = {}, hi = {};
+#pragma unroll
+            for (int jj = 0; jj < 8; ++jj) {
+                lo = mfma32(a[jj], in.lo[jj], lo);
+                hi = mfma32(a[jj], in.hi[jj], hi);
+            }
+            const float xv = in.d[0], wd = in.wd;
+            if (next < nc) load(in, next);
+            static_for<4>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                p[0][i] = row_bcast<i>(xv) * wd * static_cast<float>(lo[i] + 128 * hi[i]);  // src/quant.cpp:549-563
+            });
+        } else {
+            float dv[8], sv[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                dv[k] = in.d[q8k ? 0 : k];
+                sv[k] = kSums ? dv[k] * static_cast<float>(in.bs[T == kQ4_1 ? k : 0]) : 0.0f;
+            }
+            v4u sums = {};
+            if constexpr (T == kQ4_K) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    sums[k] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(static_cast<float>(in.bs[2 * k]), static_cast<float>(in.bs[2 * k + 1])));
+            }
+            MgWave<T>& Wl = wl[wave];
+            mg_put<T>(Wl, in.w);
+            if (next < nc) load(in, next);
+            const MgS sc = mg_scales<T>(Wl);
+            if constexpr (T == kQ4_K) {
+                v16i lo[2] = {}, hi[2] = {};  // two chains of each (exact sums: any split)
+#pragma unroll
+                for (int jp = 0; jp < 4; ++jp) {
+                    const int r = lane & 31;
+                    const v4u q = Wl.q[r * 8 + ((2 * jp + h) ^ mg_swz<T>(r))];
+#pragma unroll
+                    for (int o = 0; o < 2; ++o) {
+                        const int jj = 2 * jp + o;
+                        const v4u qn = (q >> (4u * o)) & 0x0F0F0F0Fu;
+                        const uint32_t sb = u4_word(sc.sc, jj >> 2) >> (8 * (jj & 3));
+                        lo[o] = mfma32(a[jj], mul_bytes(qn, sb & 7), lo[o]);
+                        hi[o] = mfma32(a[jj], mul_bytes(qn, (sb >> 3) & 7), hi[o]);
+                    }
+                }
+                const v16f off = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, sums), __builtin_bit_cast(v8h, mg_mins(h ? sc.sc.w : sc.sc.z)), v16f{}, 0, 0, 0);
+                const float dw = h2f(static_cast<uint16_t>(sc.mn.x & 0xFFFF)), dmin = h2f(static_cast<uint16_t>(sc.mn.x >> 16));
+                static_for<4>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int weighted = lo[0][i] + lo[1][i] + 8 * (hi[0][i] + hi[1][i]);
+                    p[0][i] = row_bcast<i>(dv[0]) * (dw * static_cast<float>(weighted) - dmin * off[i]);  // src/quant.cpp:500-521
+                });
+            } else if constexpr (T == kTQ2_0) {
+                v16i d[2] = {};
+#pragma unroll
+                for (int jj = 0; jj < 8; ++jj) d[jj & 1] = mfma32(a[jj], mg_frag<T>(Wl, sc, jj, h), d[jj & 1]);
+                const float wd = Wl.d[lane & 31];
+                static_for<4>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const float x = row_bcast<i>(dv[0]), v = static_cast<float>(d[0][i] + d[1][i]);
+                    p[0][i] = lut16 ? v * wd * x : x * wd * v;  // src/quant.cpp:789-802 / :580-596
+                });
             } else {
-                *o = v / (1.0f + ref_expf_s(-v)) * up;  // src/kernels_f32.cpp:287-289
+                auto half_at = [](const uint4& v, int jj) {
+                    const uint32_t word = u4_word(v, jj >> 1);
+                    return h2f(static_cast<uint16_t>((jj & 1) ? (word >> 16) : (word & 0xFFFF)));
+                };
+#pragma unroll
+                for (int jj = 0; jj < 8; ++jj) {
+                    const v16i d = mfma32(a[jj], mg_frag<T>(Wl, sc, jj, h), v16i{});
+                    const float wd = half_at(sc.sc, jj) * mg_unscale<T>(), wm = kSums ? half_at(sc.mn, jj) : 0.0f;
+                    static_for<4>([&](auto ic) {
+                        constexpr int i = decltype(ic)::value;
+                        const float v = row_bcast<i>(dv[jj]) * (static_cast<float>(d[i]) * wd);
+                        p[jj][i] = kSums ? v + row_bcast<i>(sv[jj]) * wm : v;  // src/quant.cpp:445-482
+                    });
+                }
             }
         }
+        // this chunk's turn: the chunks before it are in accl
+        while (__hip_atomic_load(&turn[mat], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != c) {
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = c == 0 ? 0.0f : accl[mat][i][lane];
+#pragma unroll
+        for (int k = 0; k < kTerms; ++k) {
+            if (k >= nb && kTerms > 1) break;  // past the row: no term
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] += p[k][i];
+        }
+        if (MODE != kMmPair && c + 1 == nc) break;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) accl[mat][i][lane] = acc[i];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the sums are in LDS before the turn is passed
+        if (lane == 0) __hip_atomic_store(&turn[mat], c + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    if constexpr (MODE == kMmPair) {
+        __syncthreads();
+        if (wave >= 4 || r0 + (lane & 31) > rmax) return;
+        const int t = t0 + 4 * h + wave;
+        if (t < g.ntok) ga.out[ti][static_cast<size_t>(t) * ga.ostride[ti] + row] = mg_gate(g, accl[0][wave][lane], accl[kMats - 1][wave][lane]);
+        return;
+    }
+    if (kw != (nc - 1) % W || r0 + (lane & 31) > rmax) return;  // the wave of the last chunk has the sums
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int t = t0 + 4 * h + i;
+        if (t >= g.ntok) continue;
+        float* o = ga.out[ti] + static_cast<size_t>(t) * ga.ostride[ti] + row;
+        if (MODE == kMmStore) *o = acc[i];
+        else if (MODE == kMmAdd) *o = *o + acc[i];  // h += proj (src/model.cpp:1111, :1162)
+        else *o = mg_gate(g, *o, acc[i]);
     }
 }
 
 // TWO: one launch for two store GEMMs of one activation (the same format and width; Q and K):
 // row tiles 0 .. of ga's rows, then gb's, each workgroup writing its own matrix's output.
-template <uint32_t T, int MODE, int G, bool TWO = false>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_mmk(MmArgs ga, MmArgs gb) {
-    __shared__ KqStage<T> st[2];
+template <int MODE, int G>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_mmk(MmArgs g) {
+    __shared__ KqStage st[2];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const uint32_t rta = (ga.m.rows + 63) / 64;
-    const bool second = TWO && blockIdx.x >= rta;
-    MmArgs g = ga;
-    if (second) {
-        g.m = gb.m;
-        g.out = gb.out;
-        g.ostride = gb.ostride;
-    }
-    const uint32_t rt0 = (second ? blockIdx.x - rta : blockIdx.x) * 64;
+    const uint32_t rt0 = blockIdx.x * 64;
     const int t0 = blockIdx.y * (16 * G);
     const int nc = static_cast<int>(g.m.cols / 256);
     MmAcc<G> a;
@@ -1445,13 +1587,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))
         for (int i = 0; i < 4; ++i) a.s[gi][i] = 0.0f;
     if (MODE == kMmGated) exp_tab_fill();  // ordered before the epilogue by the loop's barriers
     // two stages: chunk c + 1 is copied while chunk c is computed
-    kq_copy<T, G>(st[0], g.m, g.x, g.ntok, rt0, t0, 0);
+    kq_copy<G>(st[0], g.m, g.x, g.ntok, rt0, t0, 0);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     for (int c = 0; c < nc; ++c) {
-        if (c + 1 < nc) kq_copy<T, G>(st[(c + 1) & 1], g.m, g.x, g.ntok, rt0, t0, c + 1);
-        if constexpr (T == kQ4_K) kq_compute_fold<G>(kq_bases(lds_off(&st[c & 1])), a);
-        else kq_compute_fold6<G>(lds_off(&st[c & 1]), a);
+        if (c + 1 < nc) kq_copy<G>(st[(c + 1) & 1], g.m, g.x, g.ntok, rt0, t0, c + 1);
+        kq_compute_fold6<G>(lds_off(&st[c & 1]), a);
         __builtin_amdgcn_s_waitcnt(0);  // chunk c + 1 has landed (this wave's copies) ...
         __syncthreads();                // ... everyone's, and stage c & 1 is consumed
     }
@@ -1480,104 +1621,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))
                 } else {
                     *o = gv / (1.0f + ref_expf_s(-gv)) * v;  // src/kernels_f32.cpp:287-289
                 }
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------- Q4_K gate and up, fused
-
-// The gate and up projections of one row tile in one workgroup: both matrices' chunks are
-// staged beside one copy of the activations, and the epilogue applies the gate to the up
-// sums in registers (the pair's two launches stored the gate rows and read them back).
-// Each sum is the one k_mmk computes, in its term order, so the outputs are the same bits.
-struct KqPairStage {
-    alignas(16) uint8_t w0[64 * 128];  // gate: as KqStage<kQ4_K>
-    alignas(16) uint8_t wk[2048];
-    alignas(16) uint8_t u0[64 * 128];  // up
-    alignas(16) uint8_t uk[2048];
-    alignas(16) int8_t x[kKqTokMax * 256];
-    alignas(16) float xd[64];
-};
-
-__device__ __forceinline__ void kq_copy_w4k(uint8_t* w0, uint8_t* wk, const Packed& m, uint32_t r0, int c) {
-    const int tid = threadIdx.x, wave = tid >> 6, wave_first = tid & ~63;
-    const uint32_t nsb = m.cols / 256, rmax = m.rows - 1;
-    auto rowc = [&](int r) -> size_t {
-        const uint32_t rr = r0 + r <= rmax ? r0 + r : rmax;
-        return static_cast<size_t>(rr) * nsb + c;
-    };
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {  // 64 rows x 8 pieces
-        const int slot = k * kThreads + tid, r = slot >> 3, p = (slot & 7) ^ (r & 7);
-        dma16(m.p0 + rowc(r) * 128 + p * 16, w0 + (k * kThreads + wave_first) * 16);
-    }
-    if (wave < 2) {  // wave 0: the p1 rows, wave 1: the p2 rows
-        const int r = tid & 63;
-        dma16((wave ? m.p2 : m.p1) + rowc(r) * 16, wk + wave_first * 16);
-    }
-}
-
-template <int G>
-__device__ __forceinline__ void kq_copy_x(int8_t* xs, float* xd, const ActPlanar& x, int ntok, int t0, int c) {
-    const int tid = threadIdx.x, wave = tid >> 6, wave_first = tid & ~63;
-    auto tokc = [&](int t) -> size_t { return static_cast<size_t>(t0 + t < ntok ? t0 + t : ntok - 1); };
-    const size_t ds = x.stride / 32;
-#pragma unroll
-    for (int k = 0; k < G; ++k) {  // 16 G tokens x 16 pieces, G a thread
-        const int slot = k * kThreads + tid, t = slot >> 4, p = (slot & 15) ^ (t & 15);
-        dma16(x.qs + tokc(t) * x.stride + c * 256 + p * 16, xs + (k * kThreads + wave_first) * 16);
-    }
-    if (wave == 0) dma4(x.d + tokc(tid & (16 * G - 1)) * ds + c, xd);
-}
-
-template <int G>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_mmk_pair(MmArgs g) {
-    __shared__ KqPairStage st[2];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const uint32_t rt0 = blockIdx.x * 64;
-    const int t0 = blockIdx.y * (16 * G);
-    const int nc = static_cast<int>(g.m.cols / 256);
-    MmAcc<G> ag, au;
-#pragma unroll
-    for (int gi = 0; gi < G; ++gi)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ag.s[gi][i] = au.s[gi][i] = 0.0f;
-    exp_tab_fill();  // ordered before the epilogue by the loop's barriers
-    auto copy = [&](KqPairStage& d, int c) {
-        kq_copy_w4k(d.w0, d.wk, g.m, rt0, c);
-        kq_copy_w4k(d.u0, d.uk, g.m2, rt0, c);
-        kq_copy_x<G>(d.x, d.xd, g.x, g.ntok, t0, c);
-    };
-    copy(st[0], 0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    for (int c = 0; c < nc; ++c) {
-        if (c + 1 < nc) copy(st[(c + 1) & 1], c + 1);
-        KqPairStage& cur = st[c & 1];
-        kq_compute_fold<G>(KqBases{lds_off(cur.w0), lds_off(cur.wk), lds_off(cur.x), lds_off(cur.xd)}, ag);
-        kq_compute_fold<G>(KqBases{lds_off(cur.u0), lds_off(cur.uk), lds_off(cur.x), lds_off(cur.xd)}, au);
-        __builtin_amdgcn_s_waitcnt(0);  // chunk c + 1 has landed (this wave's copies) ...
-        __syncthreads();                // ... everyone's, and stage c & 1 is consumed
-    }
-    const uint32_t rmax = g.m.rows - 1;
-#pragma unroll
-    for (int gi = 0; gi < G; ++gi) {
-        const int t = t0 + 16 * gi + (lane & 15);
-        if (t >= g.ntok) continue;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t r = rt0 + wave * 16 + (lane >> 4) * 4 + i;
-            if (r > rmax) continue;
-            float* o = g.out + static_cast<size_t>(t) * g.ostride + r;
-            const float gv = ag.s[gi][i], v = au.s[gi][i];
-            if (g.relu2) {
-                const float q = gv > 0.0f ? gv : 0.0f;
-                *o = q * q * v;  // src/model.cpp:1134-1138
-            } else if (g.gelu) {
-                *o = gelu_mul(gv, v);  // src/kernels_f32.cpp:291-296
-            } else {
-                *o = gv / (1.0f + ref_expf_s(-gv)) * v;  // src/kernels_f32.cpp:287-289
             }
         }
     }
@@ -2627,18 +2670,36 @@ static void mmx_launch(const MmArgs& g, hipStream_t s) {
     else hipLaunchKernelGGL((k_mmx<MODE, 1, 1, KM>), dim3(tiles(1)), dim3(64), 0, s, g);
 }
 
+// The K-split kernel while its workgroups (32 rows x 8 tokens) are no more than the compute units: past that its
+// second round costs more than the chain it shortens.  Measured, in us split / k_mg (workgroups): Q4_K 2560 x
+// 2048, 6 tokens 5.9 / 14 (80; the 64-row kernel before: 9.0); 8192 x 2048 pair 10.5 / 15 (256); Q6_K 2048 x 8192,
+// 6 tokens 19 / 32 for k_mmx (64); 512 x 2048 7 / 10 (16); Q4_0 1024 x 3072, 33 tokens 12.5 / 17 (160); 8256 x
+// 1024, 5 tokens 10.1 / 7.4 (258); pair of 3072 x 1024, 33 tokens 15.6 / 11 (480); TQ2_0 2560 x 2560, 64 tokens
+// 34 / 20 (640).
+template <uint32_t T, int MODE>
+static bool mgs_launch_t(MgArgs a, int n, hipStream_t s) {
+    int rt = 0;
+    for (int i = 0; i < kMgMats; ++i) {
+        a.tiles[i] = i < n ? static_cast<int>((a.m[i].rows + 31) / 32) : 0;
+        rt += a.tiles[i];
+    }
+    const int tt = (a.a.ntok + kMgsTok - 1) / kMgsTok;
+    if (rt * tt > kKqCus) return false;
+    hipLaunchKernelGGL((k_mgs<T, MODE>), dim3(rt, tt), dim3(64 * kMgsWaves), 0, s, a);
+    return true;
+}
 // k_mg's tokens a workgroup.  A wider tile reads the weights fewer times and does an MFMA's full work (with 8
 // tokens three quarters of its rows are copies), but a launch is as long as its longest workgroup: 32 tokens
 // once that gives more workgroups than compute units, 16 once half as many, else 8.  Measured, in us at 32 / 16 /
 // 8 tokens (workgroups at 32): Q8_0 6144 x 2048, 512 tokens 45 / 51 / 78 (768); 4096 rows 28 / 34 / 48 (512);
-// Q4_0 pair of 3584 rows x 1024 30 / 36 / 50 (448); Q8_0 2048 x 6144 56 / 54 / 75 (256); Q4_0 1024 x 3584
-// 33 / 25 / 27 (128); TQ2_0 pair of 6912 x 2560, 64 tokens 19 / 17 / 20 (108); 3840 rows 11 / 10 / 9 (60);
-// Q4_0 pair of 3072 x 1024, 33 tokens 20 / 15 / 13 (48).
+// Q4_K 2560 x 2048 19 / 23 / 37 (320); Q8_0 2048 x 6144 56 / 54 / 75 (256); Q4_K 2048 x 2048 18 / 20 / 32 (256);
+// Q4_0 1024 x 3584 33 / 25 / 27 (128); TQ2_0 3840 x 2560, 64 tokens 11 / 10 / 9 (60).
 template <uint32_t T, int MODE>
 static void mg_launch_t(MgArgs a, int n, hipStream_t s) {
+    if (mgs_launch_t<T, MODE>(a, n, s)) return;
     int rt = 0;
     for (int i = 0; i < kMgMats; ++i) {
-        a.tiles[i] = i < n ? static_cast<int>((a.m[i].rows + 32 * kMgWaves - 1) / (32 * kMgWaves)) : 0;
+        a.tiles[i] = i < n ? static_cast<int>((a.m[i].rows + 32 * mg_row_waves<MODE>() - 1) / (32 * mg_row_waves<MODE>())) : 0;
         rt += a.tiles[i];
     }
     auto tt = [&](int tg) { return (a.a.ntok + 8 * tg - 1) / (8 * tg); };
@@ -2648,7 +2709,13 @@ static void mg_launch_t(MgArgs a, int n, hipStream_t s) {
     else if (tg == 2) hipLaunchKernelGGL((k_mg<T, MODE, 2>), grid, dim3(kThreads), 0, s, a);
     else hipLaunchKernelGGL((k_mg<T, MODE, 1>), grid, dim3(kThreads), 0, s, a);
 }
-static bool mg_takes(uint32_t type) { return type == kQ4_0 || type == kQ4_1 || type == kQ5_0 || type == kQ8_0 || type == kTQ2_0; }
+static bool mg_takes(const MmArgs& g) {
+    switch (g.m.type) {
+        case kQ4_0: case kQ4_1: case kQ5_0: case kQ8_0: case kTQ2_0: return true;
+        case kQ4_K: return g.qx == nullptr && g.qx2 == nullptr;
+        default: return false;
+    }
+}
 // g, or with n > 1 the n GEMMs of g[] (one format and width, the same activations), as one launch.
 template <int MODE>
 static hipError_t mg_launch(const MmArgs* g, int n, hipStream_t s) {
@@ -2665,6 +2732,7 @@ static hipError_t mg_launch(const MmArgs* g, int n, hipStream_t s) {
         case kQ5_0: mg_launch_t<kQ5_0, MODE>(a, n, s); break;
         case kQ8_0: mg_launch_t<kQ8_0, MODE>(a, n, s); break;
         case kTQ2_0: mg_launch_t<kTQ2_0, MODE>(a, n, s); break;
+        case kQ4_K: mg_launch_t<kQ4_K, MODE>(a, n, s); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -2688,18 +2756,19 @@ static hipError_t mm_dispatch(const MmArgs& g, hipStream_t s) {
                 mmx_launch<MODE, true>(g, s);
                 break;
             }
-            if (kq_g == 4) hipLaunchKernelGGL((k_mmk<kQ4_K, MODE, 4>), kq_grid, dim3(kThreads), 0, s, g, g);
-            else if (kq_g == 2) hipLaunchKernelGGL((k_mmk<kQ4_K, MODE, 2>), kq_grid, dim3(kThreads), 0, s, g, g);
-            else hipLaunchKernelGGL((k_mmk<kQ4_K, MODE, 1>), kq_grid, dim3(kThreads), 0, s, g, g);
+            return hipErrorInvalidValue;  // packed Q4_K takes k_mg
             break;
         case kQ6_K:
             if (g.qx != nullptr) {
-                mmx_launch<MODE, false>(g, s);
+                MgArgs a{};
+                a.a = g;
+                a.m[0] = g.m; a.out[0] = g.out; a.ostride[0] = g.ostride; a.qx[0] = g.qx; a.qxd[0] = g.qxd;
+                if (!mgs_launch_t<kQ6_K, MODE>(a, 1, s)) mmx_launch<MODE, false>(g, s);
                 break;
             }
-            if (kq_g == 4) hipLaunchKernelGGL((k_mmk<kQ6_K, MODE, 4>), kq_grid, dim3(kThreads), 0, s, g, g);
-            else if (kq_g == 2) hipLaunchKernelGGL((k_mmk<kQ6_K, MODE, 2>), kq_grid, dim3(kThreads), 0, s, g, g);
-            else hipLaunchKernelGGL((k_mmk<kQ6_K, MODE, 1>), kq_grid, dim3(kThreads), 0, s, g, g);
+            if (kq_g == 4) hipLaunchKernelGGL((k_mmk<MODE, 4>), kq_grid, dim3(kThreads), 0, s, g);
+            else if (kq_g == 2) hipLaunchKernelGGL((k_mmk<MODE, 2>), kq_grid, dim3(kThreads), 0, s, g);
+            else hipLaunchKernelGGL((k_mmk<MODE, 1>), kq_grid, dim3(kThreads), 0, s, g);
             break;
         default: return hipErrorInvalidValue;
     }
@@ -2714,7 +2783,7 @@ static bool pair_split() {
 
 // Rows of whole 256-value chunks; the 32-value-block formats (k_mg) also take a partial last chunk.
 static bool mm_shape_ok(const MmArgs& g) {
-    const bool small_blocks = mg_takes(g.m.type) && g.m.type != kTQ2_0;
+    const bool small_blocks = g.m.type == kQ4_0 || g.m.type == kQ4_1 || g.m.type == kQ5_0 || g.m.type == kQ8_0;
     return (g.m.cols % kChunkCols == 0 || (small_blocks && g.m.cols % 32 == 0)) && g.x.stride % kChunkCols == 0 &&
            static_cast<size_t>(g.x.stride) >= g.m.cols;
 }
@@ -2723,11 +2792,20 @@ hipError_t launch_mm(const MmArgs& g, int mode, hipStream_t s) {
     if (g.ntok <= 0) return hipSuccess;
     if (!mm_shape_ok(g)) return hipErrorInvalidValue;
     if (mode == kMmPair && (g.m2.type != g.m.type || g.m2.rows != g.m.rows || g.m2.cols != g.m.cols)) return hipErrorInvalidValue;
-    if (mg_takes(g.m.type)) {
+    if (mg_takes(g)) {
         switch (mode) {
             case kMmStore: return mg_launch<kMmStore>(&g, 1, s);
             case kMmAdd: return mg_launch<kMmAdd>(&g, 1, s);
-            case kMmPair: return mg_launch<kMmPair>(&g, 1, s);
+            case kMmPair: {
+                if (g.m.type != kQ4_K || !pair_split()) return mg_launch<kMmPair>(&g, 1, s);
+                const hipError_t e = mg_launch<kMmStore>(&g, 1, s);
+                if (e != hipSuccess) return e;
+                MgArgs up{};
+                up.a = g;
+                up.m[0] = g.m2; up.out[0] = g.out; up.ostride[0] = g.ostride;
+                mg_launch_t<kQ4_K, kMmGated>(up, 1, s);
+                return hipGetLastError();
+            }
             default: return hipErrorInvalidValue;
         }
     }
@@ -2735,16 +2813,6 @@ hipError_t launch_mm(const MmArgs& g, int mode, hipStream_t s) {
         case kMmStore: return mm_dispatch<kMmStore>(g, s);
         case kMmAdd: return mm_dispatch<kMmAdd>(g, s);
         case kMmPair: {
-            if (g.m.type == kQ4_K && g.qx == nullptr && g.qx2 == nullptr && !pair_split()) {  // one fused launch
-                const int row_tiles = static_cast<int>((g.m.rows + 63) / 64);
-                int kq_g = 4;
-                while (kq_g > 1 && row_tiles * ((g.ntok + 16 * kq_g - 1) / (16 * kq_g)) < kKqCus) kq_g /= 2;
-                const dim3 grid(row_tiles, (g.ntok + 16 * kq_g - 1) / (16 * kq_g));
-                if (kq_g == 4) hipLaunchKernelGGL(k_mmk_pair<4>, grid, dim3(kThreads), 0, s, g);
-                else if (kq_g == 2) hipLaunchKernelGGL(k_mmk_pair<2>, grid, dim3(kThreads), 0, s, g);
-                else hipLaunchKernelGGL(k_mmk_pair<1>, grid, dim3(kThreads), 0, s, g);
-                return hipGetLastError();
-            }
             // the gate rows into out, then up with the gated epilogue
             const hipError_t e = mm_dispatch<kMmStore>(g, s);
             if (e != hipSuccess) return e;
@@ -2759,36 +2827,20 @@ hipError_t launch_mm(const MmArgs& g, int mode, hipStream_t s) {
     }
 }
 
-// Two Q4_K store GEMMs of one activation and width (packed planes): one launch over both.
-static hipError_t mmk_two(const MmArgs& a, const MmArgs& b, hipStream_t s) {
-    // the widest token tile that still gives a workgroup to every CU, over both matrices' row tiles
-    const int row_tiles = static_cast<int>((a.m.rows + 63) / 64 + (b.m.rows + 63) / 64);
-    int kq_g = 4;
-    while (kq_g > 1 && row_tiles * ((a.ntok + 16 * kq_g - 1) / (16 * kq_g)) < kKqCus) kq_g /= 2;
-    const dim3 grid(row_tiles, (a.ntok + 16 * kq_g - 1) / (16 * kq_g));
-    if (kq_g == 4) hipLaunchKernelGGL((k_mmk<kQ4_K, kMmStore, 4, true>), grid, dim3(kThreads), 0, s, a, b);
-    else if (kq_g == 2) hipLaunchKernelGGL((k_mmk<kQ4_K, kMmStore, 2, true>), grid, dim3(kThreads), 0, s, a, b);
-    else hipLaunchKernelGGL((k_mmk<kQ4_K, kMmStore, 1, true>), grid, dim3(kThreads), 0, s, a, b);
-    return hipGetLastError();
-}
-
 hipError_t launch_mm_store(const MmArgs* g, int n, hipStream_t s) {
     if (n <= 0 || g[0].ntok <= 0) return hipSuccess;
-    const MmArgs &a = g[0], &b = g[n > 1 ? 1 : 0];
-    auto alike = [&](const MmArgs& o) {
-        return o.m.type == a.m.type && o.m.cols == a.m.cols && o.ntok == a.ntok && o.x.qs == a.x.qs && o.x.stride == a.x.stride;
-    };
+    const MmArgs& a = g[0];
     int k = 1;  // the first k GEMMs as one launch
-    if (mg_takes(a.m.type)) {
-        while (k < n && k < kMgMats && alike(g[k])) ++k;
-    } else if (n > 1 && a.m.type == kQ4_K && alike(b) && a.qx == nullptr && b.qx == nullptr) {
-        k = 2;
-    }
-    const bool shape_ok = mm_shape_ok(a);
+    while (k < n && k < kMgMats && g[k].m.type == a.m.type && g[k].m.cols == a.m.cols && g[k].ntok == a.ntok && g[k].x.qs == a.x.qs &&
+           g[k].x.stride == a.x.stride && mg_takes(g[k]))
+        ++k;
     hipError_t e = hipSuccess;
-    if (k == 1 || !shape_ok) e = launch_mm(a, kMmStore, s);
-    else if (mg_takes(a.m.type)) e = mg_launch<kMmStore>(g, k, s);
-    else e = mmk_two(a, b, s);
+    if (k > 1 && mg_takes(a) && mm_shape_ok(a)) {
+        e = mg_launch<kMmStore>(g, k, s);
+    } else {
+        k = 1;
+        e = launch_mm(a, kMmStore, s);
+    }
     return e != hipSuccess ? e : launch_mm_store(g + k, n - k, s);
 }
 
