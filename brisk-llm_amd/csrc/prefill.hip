@@ -2690,7 +2690,8 @@ static bool mgs_launch_t(MgArgs a, int n, hipStream_t s) {
 }
 // k_mg's tokens a workgroup.  A wider tile reads the weights fewer times and does an MFMA's full work (with 8
 // tokens three quarters of its rows are copies), but a launch is as long as its longest workgroup: 32 tokens
-// once that gives more workgroups than compute units, 16 once half as many, else 8.  Measured, in us at 32 / 16 /
+// once that gives more workgroups than compute units (Q4_K, whose decoding a wider tile shares: as many), 16
+// once half as many, else 8.  Measured, in us at 32 / 16 /
 // 8 tokens (workgroups at 32): Q8_0 6144 x 2048, 512 tokens 45 / 51 / 78 (768); 4096 rows 28 / 34 / 48 (512);
 // Q4_K 2560 x 2048 19 / 23 / 37 (320); Q8_0 2048 x 6144 56 / 54 / 75 (256); Q4_K 2048 x 2048 18 / 20 / 32 (256);
 // Q4_0 1024 x 3584 33 / 25 / 27 (128); TQ2_0 3840 x 2560, 64 tokens 11 / 10 / 9 (60).
@@ -2703,7 +2704,7 @@ static void mg_launch_t(MgArgs a, int n, hipStream_t s) {
         rt += a.tiles[i];
     }
     auto tt = [&](int tg) { return (a.a.ntok + 8 * tg - 1) / (8 * tg); };
-    const int tg = rt * tt(4) > kKqCus ? 4 : rt * tt(2) >= kKqCus / 2 ? 2 : 1;
+    const int tg = rt * tt(4) >= kKqCus + (T == kQ4_K ? 0 : 1) ? 4 : rt * tt(2) >= kKqCus / 2 ? 2 : 1;
     const dim3 grid(rt, tt(tg));
     if (tg == 4) hipLaunchKernelGGL((k_mg<T, MODE, 4>), grid, dim3(kThreads), 0, s, a);
     else if (tg == 2) hipLaunchKernelGGL((k_mg<T, MODE, 2>), grid, dim3(kThreads), 0, s, a);
