@@ -4,15 +4,14 @@
 // Exactness.  The reference multiplies block by block: per block (32 values,
 // or a K-quant sub-block) an exact int32 dot, then a float term added to the
 // row sum in block order (src/quant.cpp:445-596, matmul_generic
-// src/kernels.cpp:13-30 runs the same dot per token).  v_mfma_i32_16x16x32_i8
-// computes, for 16 rows x 16 tokens, exactly those int32 block dots (K = 32 is
-// one block), so the float epilogue here repeats the reference's term and sum
+// src/kernels.cpp:13-30 runs the same dot per token).  The MFMAs here compute
+// exactly those int32 dots (or, with a K-quant's scales folded in, its exact
+// weighted sums), so the float epilogues repeat the reference's term and sum
 // order per output and every output is bit-identical to the matvec path.
 //
-// Operand layouts of v_mfma_i32_16x16x32_i8 (wave of 64, lane l):
-//   A (16 x 32, rows x k):   lane l holds A[l % 16][8 (l / 16) .. + 7]
-//   B (32 x 16, k x tokens): lane l holds B[8 (l / 16) .. + 7][l % 16]
-//   D (16 x 16 int32):       lane l holds D[4 (l / 16) + i][l % 16], i = 0..3
+// Operand layouts (wave of 64, lane l), i8 A and B, int32 D:
+//   16x16x32: A row l % 16 and B column l % 16, k = 8 (l / 16) .. + 7; D row 4 (l / 16) + i, column l % 16
+//   32x32x32: A row l % 32 and B column l % 32, k = 16 (l / 32) .. + 15; D row 8 (i / 4) + 4 (l / 32) + i % 4, column l % 32
 //
 // Activations for the GEMMs are quantised per token into a planar layout
 // (ActPlanar): int8 values [T][cols], scales [T][cols / 32] (Q8_0: one per
