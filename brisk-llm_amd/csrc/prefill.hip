@@ -1148,7 +1148,9 @@ __device__ __forceinline__ v4u mg_mins(uint32_t m4) {
     return r;
 }
 
-// The gated output (a table is filled first: exp_tab_fill).
+// Whether a mode's epilogue gates (mg_gate reads the LDS table: the kernel fills it, exp_tab_fill, ahead of a barrier).
+template <int MODE>
+__host__ __device__ constexpr bool mg_gates() { return MODE == kMmPair || MODE == kMmGated; }
 __device__ __forceinline__ float mg_gate(const MmArgs& g, float gv, float up) {
     if (g.relu2) {
         const float q = gv > 0.0f ? gv : 0.0f;
@@ -1225,7 +1227,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, TG 
         }
     };
 
-    if (MODE == kMmPair || MODE == kMmGated) exp_tab_fill();  // ordered before the epilogue by the loop's barriers
+    if (mg_gates<MODE>()) exp_tab_fill();  // ordered before the epilogue by the loop's barriers
     MgRegs<T> w;  // the next chunk's
     Act act;
     auto load = [&](int c) {
@@ -1410,7 +1412,7 @@ __global__ __launch_bounds__(64 * kMgsWaves) __attribute__((amdgpu_waves_per_eu(
     const uint8_t* xq = reinterpret_cast<const uint8_t*>(g.x.qs) + ta * g.x.stride + 16 * h;
     const float* xd = g.x.d + ts * (g.x.stride / 32);
     if (tid < kMats) turn[tid] = 0;
-    if (MODE == kMmPair) exp_tab_fill();
+    if (mg_gates<MODE>()) exp_tab_fill();
     __syncthreads();
 
     auto load = [&](MgsIn<T>& in, int c) {
