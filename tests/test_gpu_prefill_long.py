@@ -155,3 +155,29 @@ def test_prompt_attention_row_blocks(name, first, second):
         got = [s.eval(prompt[:first])] + ([s.eval(prompt[first:])] if second else [])
     for g, w in zip(got, want):
         np.testing.assert_array_equal(g.view(np.uint32), w.view(np.uint32))
+
+
+@pytest.mark.parametrize("first", [40, 600])
+def test_values_outside_a_window_are_not_touched(first, tmp_path):
+    """Infinite cached values at positions that a sliding layer's token no longer sees leave it alone, also
+    where they lie beside its window or in that of an earlier row of the same block: one sliding layer
+    (8 positions), so a row's logits depend on its own window only, against the oracle bit for bit."""
+    import dataclasses
+    from test_gpu_long_context import prefill_kv, _h2d
+    spec = dataclasses.replace(synth.SPECS["tiny-gemma3"], name="one-sliding-layer", layers=1)
+    f, cfg, table = model.load(synth.write_model(spec, str(tmp_path / "m.gguf")))
+    prompt = synth.prompt_ids(33, cfg.vocab, seed=3)
+    print(f"[prefill] one sliding layer: 33 ids after {first}", flush=True)
+    o = pyoracle.Oracle(cfg, table, first + 40)
+    with HipSession((f, cfg, table), max_context=first + 40) as s:
+        prefill_kv(s, o, cfg, first, seed=8)
+        clean = o.eval(prompt, all_logits=True)
+        o.rollback(first)
+        cache = o.kv(0, True)
+        cache[:, :first - 6] = 0x7C00  # the first token sees one of them, position first - 7
+        _h2d(s.kv_cache(0, True)[0], np.ascontiguousarray(cache), cache.nbytes)
+        want, got = o.eval(prompt, all_logits=True), s.eval_all(prompt)
+    o.close()
+    assert (want[0] != clean[0]).any()
+    np.testing.assert_array_equal(want[1:], clean[1:])
+    np.testing.assert_array_equal(got[1:].view(np.uint32), want[1:].view(np.uint32))
