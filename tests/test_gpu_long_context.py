@@ -192,3 +192,31 @@ def test_spread_attention_over_many_chunks_repeats():
         np.testing.assert_array_equal(runs[k][0].view(np.uint32), runs[0][0].view(np.uint32))
         for a, b in zip(runs[k][1], runs[0][1]):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("n_pos,n", [(10000, 260), (20000, 5), (39798, 6), (39798, 7)])
+def test_prompts_late_in_a_long_context(tmp_path, n_pos, n):
+    """The prompt attention keeps its rows' scores in LDS (k_pre_attn_rows): 2 rows a workgroup past 9852
+    positions, 1 past 19836, none past 39804 (there the tokens go one by one).  Over a pre-filled cache, the
+    second layer's cached rows (from every row of the first layer's attention) and the logits against the
+    oracle bit for bit."""
+    import ctypes as C
+    import dataclasses
+    spec = dataclasses.replace(synth.SPECS["tiny-qwen3-long"], name="longer", context=40960)
+    f, cfg, table = model.load(synth.write_model(spec, str(tmp_path / "m.gguf")))
+    print(f"[long] {n} prompt ids after {n_pos} positions", flush=True)
+    prompt = synth.prompt_ids(n, cfg.vocab, seed=6)
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    with HipSession((f, cfg, table), max_context=n_pos + n + 8) as s:
+        o = pyoracle.Oracle(cfg, table, n_pos + n + 8)
+        prefill_kv(s, o, cfg, n_pos, seed=12)
+        got, want = s.eval(prompt), o.eval(prompt)
+        for value in (False, True):
+            ptr, nbytes = s.kv_cache(1, value)
+            host = np.empty(nbytes // 2, np.uint16)
+            assert hip.hipMemcpy(C.c_void_p(host.ctypes.data), C.c_void_p(ptr), nbytes, 2) == 0  # hipMemcpyDeviceToHost
+            rows = slice(n_pos, n_pos + n)
+            np.testing.assert_array_equal(host.reshape(cfg.kv_heads, -1, cfg.head_dim)[:, rows], o.kv(1, value)[:, rows])
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+        o.close()

@@ -88,6 +88,7 @@ def test_mfma_attention_tiny(name):
 
 
 @pytest.mark.slow
+@pytest.mark.skipif(not pyoracle.ref_available(), reason="oracle/_ref/libbrisk_ref.so is not built (no reference tree)")
 def test_mfma_attention_llama_512():
     """configs[2] (Llama-3.2-1B-shape Q4_K_M), 512-token prompt against the
     reference engine: the default path bit for bit, the opt-in MFMA attention
@@ -181,3 +182,21 @@ def test_values_outside_a_window_are_not_touched(first, tmp_path):
     assert (want[0] != clean[0]).any()
     np.testing.assert_array_equal(want[1:], clean[1:])
     np.testing.assert_array_equal(got[1:].view(np.uint32), want[1:].view(np.uint32))
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(14, 2, 64), (6, 2, 128), (15, 1, 64)])
+def test_query_heads_that_do_not_divide_a_row_block(heads, kv_heads, head_dim, tmp_path):
+    """7, 3 and 15 query heads a key/value head: blocks of rows begin and end inside a token's heads, at each
+    number of rows a workgroup, from the start of a sequence and continued."""
+    import dataclasses
+    spec = dataclasses.replace(synth.SPECS["tiny-qwen3-long"], name="odd-heads", heads=heads, kv_heads=kv_heads, head_dim=head_dim)
+    f, cfg, table = model.load(synth.write_model(spec, str(tmp_path / "m.gguf")))
+    prompt = synth.prompt_ids(620, cfg.vocab, seed=19)
+    cuts = (0, 2, 7, 40, 330, 333, 620)
+    print(f"[prefill] {heads} query heads, {kv_heads} kv heads of {head_dim}", flush=True)
+    o = pyoracle.Oracle(cfg, table, 632)
+    with HipSession((f, cfg, table), max_context=632) as s:
+        for a, b in zip(cuts, cuts[1:]):
+            got, want = s.eval(prompt[a:b]), o.eval(prompt[a:b])
+            np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32), err_msg=f"ids {a}..{b}")
+    o.close()
