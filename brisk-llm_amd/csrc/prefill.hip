@@ -420,28 +420,28 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 2))
     }
 }
 
-// ---------------------------------------------------------------- the packed Q6_K GEMM, staged through LDS
+// ---------------------------------------------------------------- the packed Q4_K / Q6_K GEMM, staged through LDS
 
-// Q6_K without expanded planes (one 256-value super-block a row per chunk).  A workgroup of 4
-// waves computes 64 rows x 32 tokens; wave w owns rows 16 w .. + 15 for the
-// 32 tokens (2 groups of 16).  Per chunk every operand -- the 64 rows' weight
-// planes and the 32 tokens' int8 values, bsums and scales -- is copied global
-// -> LDS by global_load_lds (16 bytes a lane, no registers held), and the
-// waves read their MFMA fragments from there.  The stage is small (22 KB) and
-// the registers few, so several workgroups share a CU and one's copies overlap
-// the others' MFMAs.  The arithmetic is wchunk_compute's: exact int32 block
-// dots, the reference's float term and sum order.
+// Q4_K, and Q6_K without expanded planes (one 256-value super-block a row per chunk).  A
+// workgroup of 4 waves computes 64 rows x 16 G tokens; wave w owns rows 16 w .. + 15 for
+// the G groups of 16 tokens.  Per chunk every operand -- the 64 rows' weight planes and
+// the tokens' int8 values and scales -- is copied global -> LDS by global_load_lds (16
+// bytes a lane, no registers held), and the waves read their MFMA fragments from there.
+// The stage is small (27 or 30 KB) and the registers few, so workgroups share a CU and
+// one's copies overlap the others' MFMAs.  The arithmetic: exact int32 sums, the
+// reference's float term and sum order.
 constexpr int kKqTokMax = 64;
 constexpr int kKqCus = 256;  // MI355X compute units (the tile choice aims at a workgroup each)
 // tokens a workgroup: 16 G (G token groups share each weight fragment's decode); the
 // launcher takes the largest G that still gives a workgroup to every CU
 
+template <uint32_t T>
 struct KqStage {
-    alignas(16) uint8_t w0[64 * 128];         // ql: row r piece p at slot r * 8 + (p ^ (r & 7))
-    alignas(16) uint8_t wk[4096];             // qh: row r piece p at r * 4 + (p ^ (r & 3))
-    alignas(16) uint32_t wm[384];             // the 20-byte meta of row r at dwords 5 r .. 5 r + 4
-    alignas(16) int8_t x[kKqTokMax * 256];    // token t piece p at slot t * 16 + (p ^ (t & 15))
-    alignas(16) float xd[64];                 // Q8_K scale of token t (lanes 32..63: a copy)
+    alignas(16) uint8_t w0[64 * 128];                  // Q4_K nibbles / Q6_K ql: row r piece p at slot r * 8 + (p ^ (r & 7))
+    alignas(16) uint8_t wk[T == kQ4_K ? 2048 : 4096];  // Q4_K: p1 [64][16] then p2 [64][16]; Q6_K: qh, row r piece p at r * 4 + (p ^ (r & 3))
+    alignas(16) uint32_t wm[T == kQ6_K ? 384 : 1];     // Q6_K: the 20-byte meta of row r at dwords 5 r .. 5 r + 4
+    alignas(16) int8_t x[kKqTokMax * 256];             // token t piece p at slot t * 16 + (p ^ (t & 15))
+    alignas(16) float xd[64];                          // Q8_K scale of token t (lanes past the tokens: copies)
 };
 
 __device__ __forceinline__ void dma16(const void* src, void* lds_wave_base) {
@@ -451,10 +451,10 @@ __device__ __forceinline__ void dma4(const void* src, void* lds_wave_base) {
     __builtin_amdgcn_global_load_lds((global_cvoid_ptr)src, (lds_void_ptr)lds_wave_base, 4, 0, 0);
 }
 
-// Copies chunk c of rows r0 .. r0 + 63 and tokens t0 .. t0 + 31 into the stage
+// Copies chunk c of rows r0 .. r0 + 63 and tokens t0 .. t0 + 16 G - 1 into the stage
 // (rows and tokens past the ends re-read the last one; their outputs are not stored).
-template <int G>
-__device__ __forceinline__ void kq_copy(KqStage& st, const Packed& m, const ActPlanar& x, int ntok, uint32_t r0, int t0, int c) {
+template <uint32_t T, int G>
+__device__ __forceinline__ void kq_copy(KqStage<T>& st, const Packed& m, const ActPlanar& x, int ntok, uint32_t r0, int t0, int c) {
     const int tid = threadIdx.x, wave = tid >> 6, wave_first = tid & ~63;
     const uint32_t nsb = m.cols / 256, rmax = m.rows - 1;
     auto rowc = [&](int r) -> size_t {
@@ -467,16 +467,21 @@ __device__ __forceinline__ void kq_copy(KqStage& st, const Packed& m, const ActP
         const int slot = k * kThreads + tid, r = slot >> 3, p = (slot & 7) ^ (r & 7);
         dma16(m.p0 + rowc(r) * 128 + p * 16, st.w0 + (k * kThreads + wave_first) * 16);
     }
-    {  // qh: 64 rows x 4 pieces; meta: 320 dwords
+    if (T == kQ4_K) {  // wave 0: the p1 rows, wave 1: the p2 rows
+        if (wave < 2) {
+            const int r = tid & 63;
+            dma16((wave ? m.p2 : m.p1) + rowc(r) * 16, st.wk + wave_first * 16);
+        }
+    } else {  // qh: 64 rows x 4 pieces; meta: 320 dwords
         const int r = tid >> 2, p = (tid & 3) ^ (r & 3);
         dma16(m.p1 + rowc(r) * 64 + p * 16, st.wk + wave_first * 16);
-    }
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int slot = k * kThreads + tid;
-        if (slot < 384) {  // waves of slots 320..383 copy row 63's meta again into the spare
-            const int sl = slot < 320 ? slot : 319, r2 = sl / 5, j = sl - r2 * 5;
-            dma4(m.p2 + rowc(r2) * 20 + j * 4, st.wm + k * kThreads + wave_first);
+        for (int k = 0; k < 2; ++k) {
+            const int slot = k * kThreads + tid;
+            if (slot < 384) {  // waves of slots 320..383 copy row 63's meta again into the spare
+                const int sl = slot < 320 ? slot : 319, r2 = sl / 5, j = sl - r2 * 5;
+                dma4(m.p2 + rowc(r2) * 20 + j * 4, st.wm + k * kThreads + wave_first);
+            }
         }
     }
     const size_t ds = x.stride / 32;
@@ -535,6 +540,113 @@ __device__ __forceinline__ v4u mul_bytes(const v4u& q, uint32_t d) {
     return v4u{mul_bytes1(q.x, dd), mul_bytes1(q.y, dd), mul_bytes1(q.z, dd), mul_bytes1(q.w, dd)};
 }
 
+// Q4_K with the scales folded into the MFMAs.  For sub-block j of a row,
+// weighted = sum_j sc_j dot_j and offsets = sum_j mn_j pair_j (dot_q4_k_q8_k,
+// src/quant.cpp:500-521) are exact integers; with sc_j = lo_j + 8 hi_j (3-bit
+// digits) and q in 0..15, q lo_j and q hi_j fit int8, so
+//   weighted = A_lo + 8 A_hi,  A_lo = sum_k (q_k lo_j(k)) x_k,  A_hi likewise,
+//   offsets  = sum_k mn_j(k) x_k   (pair_j is the sum of sub-block j's x),
+// three int32 MFMA chains over the super-block (mfma64: lanes 0..31 are sub-block
+// 2 s and lanes 32..63 sub-block 2 s + 1 of step s, and each lane's digit is its own
+// sub-block's).  The float term per super-block is the reference's.
+
+// LDS addresses of a Q4_K stage's parts: the nibble rows, the {d, dmin, scales} and decoded
+// scale/min rows (wk, then wk + 1024), the activations and their scales.
+struct KqBases {
+    uint32_t w0, wk, x, xd;
+};
+__device__ __forceinline__ KqBases kq_bases(uint32_t base) {
+    return KqBases{base + static_cast<uint32_t>(offsetof(KqStage<kQ4_K>, w0)), base + static_cast<uint32_t>(offsetof(KqStage<kQ4_K>, wk)),
+                   base + static_cast<uint32_t>(offsetof(KqStage<kQ4_K>, x)), base + static_cast<uint32_t>(offsetof(KqStage<kQ4_K>, xd))};
+}
+
+// Fragments read by kq_f64_issue; kq_f64_wait ties each as one 128-bit operand,
+// so no copy of a fragment register can be placed before the wait.
+struct KqF64 {
+    v4u a, b0, b1, b2, b3;  // b0 .. b(G-1) used
+};
+template <int G>
+__device__ __forceinline__ KqF64 kq_f64_issue(const KqBases& b, int s, int ar, int tl, int l16) {
+    KqF64 f;
+    const int pa = 2 * s + (l16 & 1);  // Q4_K: 32 bytes of nibbles a sub-block pair, low then high
+    f.a = ds128v(b.w0 + (ar * 8 + (pa ^ (ar & 7))) * 16);
+    const int pb = 4 * s + l16;
+    auto bfrag = [&](int g) -> v4u {
+        const int t = 16 * g + tl;
+        return ds128v(b.x + (t * 16 + (pb ^ (t & 15))) * 16);
+    };
+    const v4u z = {0u, 0u, 0u, 0u};
+    f.b0 = bfrag(0);
+    f.b1 = G > 1 ? bfrag(1) : z;
+    f.b2 = G > 2 ? bfrag(2) : z;
+    f.b3 = G > 3 ? bfrag(3) : z;
+    return f;
+}
+__device__ __forceinline__ void kq_f64_wait(KqF64& f) {
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f.a), "+v"(f.b0), "+v"(f.b1), "+v"(f.b2), "+v"(f.b3));
+}
+
+template <int G>
+__device__ __forceinline__ void kq_compute_fold(const KqBases& base, MmAcc<G>& acc) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tl = lane & 15, l16 = lane >> 4;
+    const int ar = wave * 16 + tl, orow0 = wave * 16 + l16 * 4;
+    const v4i zero = {0, 0, 0, 0};
+    // the A row's decoded scales and mins (for the digits), the output rows' d / dmin, the groups' x scales
+    v4u scm = ds128v(base.wk + 1024 + ar * 16);
+    uint32_t dd[4], xd[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        dd[i] = ds32(base.wk + (orow0 + i) * 16);
+        xd[i] = i < G ? ds32(base.xd + (16 * i + tl) * 4) : 0u;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(scm), "+v"(dd[0]), "+v"(dd[1]), "+v"(dd[2]), "+v"(dd[3]), "+v"(xd[0]), "+v"(xd[1]), "+v"(xd[2]),
+                   "+v"(xd[3]));
+    KqF64 cur = kq_f64_issue<G>(base, 0, ar, tl, l16);
+    kq_f64_wait(cur);
+    v4i alo[4], ahi[4], amn[4];
+#pragma unroll
+    for (int g = 0; g < G; ++g) alo[g] = ahi[g] = amn[g] = zero;
+    // lanes 32..63 take the odd sub-block of the pair (high nibbles): a shift by 4, not a select
+    const uint32_t nib_shift = l16 >= 2 ? 4u : 0u;
+    const uint32_t lane_byte = static_cast<uint32_t>(l16 >> 1) * 0x01010101u;
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+        KqF64 nxt;
+        if (st < 3) nxt = kq_f64_issue<G>(base, st + 1, ar, tl, l16);
+        const int j = 2 * st + (l16 >> 1);  // this lane's sub-block (j < 4 exactly when st < 2)
+        const uint32_t sc = ((st < 2 ? scm.x : scm.y) >> (8 * (j & 3))) & 0xFF;
+        // the min byte of sub-block j in all four bytes (v_perm_b32: byte j & 3 of the word, four times)
+        const uint32_t m4 = __builtin_amdgcn_perm(0u, st < 2 ? scm.z : scm.w, lane_byte + static_cast<uint32_t>((2 * st) & 3) * 0x01010101u);
+        const uint32_t dlo = sc & 7, dhi = sc >> 3;
+        const v4u qn = (cur.a >> nib_shift) & 0x0F0F0F0Fu;
+        const v4u qlo = mul_bytes(qn, dlo);  // bytes 0..15 times 0..7: no carries between bytes
+        const v4u qhi = mul_bytes(qn, dhi);
+        const v4u qmn = {m4, m4, m4, m4};
+        const v4u bq[4] = {cur.b0, cur.b1, cur.b2, cur.b3};
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            alo[g] = mfma64(qlo, bq[g], alo[g]);
+            ahi[g] = mfma64(qhi, bq[g], ahi[g]);
+            amn[g] = mfma64(qmn, bq[g], amn[g]);
+        }
+        if (st < 3) {
+            kq_f64_wait(nxt);
+            cur = nxt;
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const float xg = __uint_as_float(xd[g]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int weighted = alo[g][i] + 8 * ahi[g][i], offsets = amn[g][i];
+            const float d = h2f(static_cast<uint16_t>(dd[i] & 0xFFFF)), dmin = h2f(static_cast<uint16_t>(dd[i] >> 16));
+            acc.s[g][i] += xg * (d * static_cast<float>(weighted) - dmin * static_cast<float>(offsets));  // src/quant.cpp:500-521
+        }
+    }
+}
+
 // Q6_K with its signed 8-bit scales folded into the MFMAs.  Per 16-value
 // group g of a super-block, weighted = sum_g sc_g dot_g with dot_g = sum (q - 32) x
 // (dot_q6_k_q8_k, src/quant.cpp:549-563).  With sc_g + 128 = sum_i 4^i d_i,g
@@ -559,12 +671,12 @@ __device__ __forceinline__ Kq6F kq6_issue(uint32_t base, int st, int ar, int tl,
     Kq6F f;
     const int half = st >> 1;
     const int lp = half * 4 + l16, hp = half * 2 + (l16 & 1);
-    f.l = ds128v(base + offsetof(KqStage, w0) + (ar * 8 + (lp ^ (ar & 7))) * 16);
-    f.h = ds128v(base + offsetof(KqStage, wk) + (ar * 4 + (hp ^ (ar & 3))) * 16);
+    f.l = ds128v(base + offsetof(KqStage<kQ6_K>, w0) + (ar * 8 + (lp ^ (ar & 7))) * 16);
+    f.h = ds128v(base + offsetof(KqStage<kQ6_K>, wk) + (ar * 4 + (hp ^ (ar & 3))) * 16);
     const int pb = 4 * st + l16;
     auto bfrag = [&](int g) -> v4u {
         const int t = 16 * g + tl;
-        return ds128v(base + offsetof(KqStage, x) + (t * 16 + (pb ^ (t & 15))) * 16);
+        return ds128v(base + offsetof(KqStage<kQ6_K>, x) + (t * 16 + (pb ^ (t & 15))) * 16);
     };
     const v4u z = {0u, 0u, 0u, 0u};
     f.b0 = bfrag(0);
@@ -583,13 +695,13 @@ __device__ __forceinline__ void kq_compute_fold6(uint32_t base, MmAcc<G>& acc) {
     const int ar = wave * 16 + tl, orow0 = wave * 16 + l16 * 4;
     const v4i zero = {0, 0, 0, 0};
     // the A row's 16 int8 scales (four dwords of its meta), the output rows' d, the groups' x scales
-    const uint32_t arow = base + offsetof(KqStage, wm) + ar * 20;
+    const uint32_t arow = base + offsetof(KqStage<kQ6_K>, wm) + ar * 20;
     uint32_t s0 = ds32(arow), s1 = ds32(arow + 4), s2 = ds32(arow + 8), s3 = ds32(arow + 12);
     uint32_t dd[4], xd[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        dd[i] = ds32(base + offsetof(KqStage, wm) + (orow0 + i) * 20 + 16);
-        xd[i] = i < G ? ds32(base + offsetof(KqStage, xd) + (16 * i + tl) * 4) : 0u;
+        dd[i] = ds32(base + offsetof(KqStage<kQ6_K>, wm) + (orow0 + i) * 20 + 16);
+        xd[i] = i < G ? ds32(base + offsetof(KqStage<kQ6_K>, xd) + (16 * i + tl) * 4) : 0u;
     }
     asm volatile("s_waitcnt lgkmcnt(0)"
                  : "+v"(s0), "+v"(s1), "+v"(s2), "+v"(s3), "+v"(dd[0]), "+v"(dd[1]), "+v"(dd[2]), "+v"(dd[3]), "+v"(xd[0]),
@@ -1572,32 +1684,38 @@ __global__ __launch_bounds__(64 * kMgsWaves) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
-// TWO: one launch for two store GEMMs of one activation (the same format and width; Q and K):
-// row tiles 0 .. of ga's rows, then gb's, each workgroup writing its own matrix's output.
-template <int MODE, int G>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_mmk(MmArgs g) {
-    __shared__ KqStage st[2];
+// The packed-plane GEMM of Q4_K and Q6_K.  MANY: up to kMgMats matrices of one format and width (64-row tiles of
+// each); apart from the one-matrix form because finding the tile's matrix takes 0.4 us of a 9 us launch.
+template <uint32_t T, int MODE, int G, bool MANY>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_mmk(MgArgs ga) {
+    __shared__ KqStage<T> st[2];
+    const MmArgs& g = ga.a;
+    int tile = blockIdx.x, ti = 0;
+    if (MANY)
+        while (ti < kMgMats - 1 && tile >= ga.tiles[ti]) tile -= ga.tiles[ti++];
+    const Packed m = ga.m[ti];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const uint32_t rt0 = blockIdx.x * 64;
+    const uint32_t rt0 = static_cast<uint32_t>(tile) * 64;
     const int t0 = blockIdx.y * (16 * G);
-    const int nc = static_cast<int>(g.m.cols / 256);
+    const int nc = static_cast<int>(m.cols / 256);
     MmAcc<G> a;
 #pragma unroll
     for (int gi = 0; gi < G; ++gi)
 #pragma unroll
         for (int i = 0; i < 4; ++i) a.s[gi][i] = 0.0f;
-    if (MODE == kMmGated) exp_tab_fill();  // ordered before the epilogue by the loop's barriers
+    if (mg_gates<MODE>()) exp_tab_fill();  // ordered before the epilogue by the loop's barriers
     // two stages: chunk c + 1 is copied while chunk c is computed
-    kq_copy<G>(st[0], g.m, g.x, g.ntok, rt0, t0, 0);
+    kq_copy<T, G>(st[0], m, g.x, g.ntok, rt0, t0, 0);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     for (int c = 0; c < nc; ++c) {
-        if (c + 1 < nc) kq_copy<G>(st[(c + 1) & 1], g.m, g.x, g.ntok, rt0, t0, c + 1);
-        kq_compute_fold6<G>(lds_off(&st[c & 1]), a);
+        if (c + 1 < nc) kq_copy<T, G>(st[(c + 1) & 1], m, g.x, g.ntok, rt0, t0, c + 1);
+        if constexpr (T == kQ4_K) kq_compute_fold<G>(kq_bases(lds_off(&st[c & 1])), a);
+        else kq_compute_fold6<G>(lds_off(&st[c & 1]), a);
         __builtin_amdgcn_s_waitcnt(0);  // chunk c + 1 has landed (this wave's copies) ...
         __syncthreads();                // ... everyone's, and stage c & 1 is consumed
     }
-    const uint32_t rmax = g.m.rows - 1;
+    const uint32_t rmax = m.rows - 1;
 #pragma unroll
     for (int gi = 0; gi < G; ++gi) {
         const int t = t0 + 16 * gi + (lane & 15);
@@ -1606,23 +1724,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))
         for (int i = 0; i < 4; ++i) {
             const uint32_t r = rt0 + wave * 16 + (lane >> 4) * 4 + i;
             if (r > rmax) continue;
-            float* o = g.out + static_cast<size_t>(t) * g.ostride + r;
+            float* o = ga.out[ti] + static_cast<size_t>(t) * ga.ostride[ti] + r;
             const float v = a.s[gi][i];
-            if (MODE == kMmStore) {
-                *o = v;
-            } else if (MODE == kMmAdd) {
-                *o = *o + v;  // h += proj (src/model.cpp:1111, :1162)
-            } else {  // kMmGated: out holds the gate row, this is up
-                const float gv = *o;
-                if (g.relu2) {
-                    const float q = gv > 0.0f ? gv : 0.0f;
-                    *o = q * q * v;  // src/model.cpp:1134-1138
-                } else if (g.gelu) {
-                    *o = gelu_mul(gv, v);  // src/kernels_f32.cpp:291-296
-                } else {
-                    *o = gv / (1.0f + ref_expf_s(-gv)) * v;  // src/kernels_f32.cpp:287-289
-                }
-            }
+            if (MODE == kMmStore) *o = v;
+            else if (MODE == kMmAdd) *o = *o + v;  // h += proj (src/model.cpp:1111, :1162)
+            else *o = mg_gate(g, *o, v);           // kMmGated: out holds the gate row, this is up
         }
     }
 }
@@ -2686,6 +2792,33 @@ static void mmx_launch(const MmArgs& g, hipStream_t s) {
     else hipLaunchKernelGGL((k_mmx<MODE, 1, 1, KM>), dim3(tiles(1)), dim3(64), 0, s, g);
 }
 
+// The first n matrices' tiles of `rows` rows into a.tiles; their number.
+static int mg_tiles(MgArgs& a, int n, int rows) {
+    int rt = 0;
+    for (int i = 0; i < kMgMats; ++i) {
+        a.tiles[i] = i < n ? (static_cast<int>(a.m[i].rows) + rows - 1) / rows : 0;
+        rt += a.tiles[i];
+    }
+    return rt;
+}
+
+// k_mmk with the most token groups, up to GMAX, that still give every compute unit a workgroup and have tokens.
+template <uint32_t T, int MODE, int GMAX, bool MANY>
+static void kq_launch_n(const MgArgs& a, int rt, hipStream_t s) {
+    auto tt = [&](int gr) { return (a.a.ntok + 16 * gr - 1) / (16 * gr); };
+    if (GMAX > 2 && a.a.ntok > 32 && rt * tt(4) >= kKqCus) hipLaunchKernelGGL((k_mmk<T, MODE, GMAX, MANY>), dim3(rt, tt(4)), dim3(kThreads), 0, s, a);
+    else if (a.a.ntok > 16 && rt * tt(2) >= kKqCus) hipLaunchKernelGGL((k_mmk<T, MODE, 2, MANY>), dim3(rt, tt(2)), dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL((k_mmk<T, MODE, 1, MANY>), dim3(rt, tt(1)), dim3(kThreads), 0, s, a);
+}
+template <uint32_t T, int MODE, int GMAX>
+static void kq_launch(MgArgs a, int n, hipStream_t s) {
+    const int rt = mg_tiles(a, n, 64);
+    if constexpr (T == kQ4_K && MODE == kMmStore) {
+        if (n > 1) return kq_launch_n<T, MODE, GMAX, true>(a, rt, s);
+    }
+    kq_launch_n<T, MODE, GMAX, false>(a, rt, s);
+}
+
 // The K-split kernel while its workgroups (32 rows x 8 tokens) are no more than the compute units: past that its
 // second round costs more than the chain it shortens.  Measured, in us split / k_mg (workgroups): Q4_K 2560 x
 // 2048, 6 tokens 5.9 / 14 (80; the 64-row kernel before: 9.0); 8192 x 2048 pair 10.5 / 15 (256); Q6_K 2048 x 8192,
@@ -2694,11 +2827,7 @@ static void mmx_launch(const MmArgs& g, hipStream_t s) {
 // 34 / 20 (640).
 template <uint32_t T, int MODE>
 static bool mgs_launch_t(MgArgs a, int n, hipStream_t s) {
-    int rt = 0;
-    for (int i = 0; i < kMgMats; ++i) {
-        a.tiles[i] = i < n ? static_cast<int>((a.m[i].rows + 31) / 32) : 0;
-        rt += a.tiles[i];
-    }
+    const int rt = mg_tiles(a, n, 32);
     const int tt = (a.a.ntok + kMgsTok - 1) / kMgsTok;
     if (rt * tt > kKqCus) return false;
     hipLaunchKernelGGL((k_mgs<T, MODE>), dim3(rt, tt), dim3(64 * kMgsWaves), 0, s, a);
@@ -2711,20 +2840,25 @@ static bool mgs_launch_t(MgArgs a, int n, hipStream_t s) {
 // 8 tokens (workgroups at 32): Q8_0 6144 x 2048, 512 tokens 45 / 51 / 78 (768); 4096 rows 28 / 34 / 48 (512);
 // Q4_K 2560 x 2048 19 / 23 / 37 (320); Q8_0 2048 x 6144 56 / 54 / 75 (256); Q4_K 2048 x 2048 18 / 20 / 32 (256);
 // Q4_0 1024 x 3584 33 / 25 / 27 (128); TQ2_0 3840 x 2560, 64 tokens 11 / 10 / 9 (60).
+// Q4_K that is not a pair takes k_mg at 32 tokens or k_mmk (64 rows x 16 or 32 tokens, whose MFMAs have no copied
+// rows): in us k_mmk / k_mg at 8 or 16 tokens, 2048 x 8192, 64 tokens 27.5 / 35.3; 8192 x 2048, 9 tokens 11.6 / 13.7;
+// 2560 x 2560, 64 tokens 13.3 / 15.6, 256 tokens 20.9 / 23.2; 12000 x 1024, 33 tokens 11.9 / 14.4; 300 x 4096, 512
+// tokens 19.3 / 23.5; with the 32-token tile, 2560 x 2048 as two matrices, 512 tokens 20.3 / 18.1.
 template <uint32_t T, int MODE>
 static void mg_launch_t(MgArgs a, int n, hipStream_t s) {
     if (mgs_launch_t<T, MODE>(a, n, s)) return;
-    int rt = 0;
-    for (int i = 0; i < kMgMats; ++i) {
-        a.tiles[i] = i < n ? static_cast<int>((a.m[i].rows + 32 * mg_row_waves<MODE>() - 1) / (32 * mg_row_waves<MODE>())) : 0;
-        rt += a.tiles[i];
-    }
+    const int rt = mg_tiles(a, n, 32 * mg_row_waves<MODE>());
     auto tt = [&](int tg) { return (a.a.ntok + 8 * tg - 1) / (8 * tg); };
-    const int tg = rt * tt(4) >= kKqCus + (T == kQ4_K ? 0 : 1) ? 4 : rt * tt(2) >= kKqCus / 2 ? 2 : 1;
-    const dim3 grid(rt, tt(tg));
-    if (tg == 4) hipLaunchKernelGGL((k_mg<T, MODE, 4>), grid, dim3(kThreads), 0, s, a);
-    else if (tg == 2) hipLaunchKernelGGL((k_mg<T, MODE, 2>), grid, dim3(kThreads), 0, s, a);
-    else hipLaunchKernelGGL((k_mg<T, MODE, 1>), grid, dim3(kThreads), 0, s, a);
+    if constexpr (T == kQ4_K && MODE != kMmPair) {
+        if (rt * tt(4) >= kKqCus) hipLaunchKernelGGL((k_mg<T, MODE, 4>), dim3(rt, tt(4)), dim3(kThreads), 0, s, a);
+        else kq_launch<T, MODE, 2>(a, n, s);
+    } else {
+        const int tg = rt * tt(4) >= kKqCus + (T == kQ4_K ? 0 : 1) ? 4 : rt * tt(2) >= kKqCus / 2 ? 2 : 1;
+        const dim3 grid(rt, tt(tg));
+        if (tg == 4) hipLaunchKernelGGL((k_mg<T, MODE, 4>), grid, dim3(kThreads), 0, s, a);
+        else if (tg == 2) hipLaunchKernelGGL((k_mg<T, MODE, 2>), grid, dim3(kThreads), 0, s, a);
+        else hipLaunchKernelGGL((k_mg<T, MODE, 1>), grid, dim3(kThreads), 0, s, a);
+    }
 }
 static bool mg_takes(const MmArgs& g) {
     switch (g.m.type) {
@@ -2758,11 +2892,6 @@ static hipError_t mg_launch(const MmArgs* g, int n, hipStream_t s) {
 template <int MODE>
 static hipError_t mm_dispatch(const MmArgs& g, hipStream_t s) {
     const dim3 grid((g.m.rows + kRowsPerWg - 1) / kRowsPerWg, (g.ntok + kQ5Tok - 1) / kQ5Tok);
-    // K-quants: the widest token tile (64, 32 or 16 tokens) that still gives a workgroup to every CU
-    const int row_tiles = static_cast<int>((g.m.rows + 63) / 64);
-    int kq_g = 4;
-    while (kq_g > 1 && row_tiles * ((g.ntok + 16 * kq_g - 1) / (16 * kq_g)) < kKqCus) kq_g /= 2;
-    const dim3 kq_grid(row_tiles, (g.ntok + 16 * kq_g - 1) / (16 * kq_g));
     switch (g.m.type) {
         case kQ5_K:
             if (g.qx != nullptr) mmx_launch<MODE, true>(g, s);
@@ -2773,20 +2902,15 @@ static hipError_t mm_dispatch(const MmArgs& g, hipStream_t s) {
                 mmx_launch<MODE, true>(g, s);
                 break;
             }
-            return hipErrorInvalidValue;  // packed Q4_K takes k_mg
+            return hipErrorInvalidValue;  // packed Q4_K: mg_launch
+        case kQ6_K: {
+            MgArgs a{};
+            a.a = g;
+            a.m[0] = g.m; a.out[0] = g.out; a.ostride[0] = g.ostride; a.qx[0] = g.qx; a.qxd[0] = g.qxd;
+            if (g.qx == nullptr) kq_launch<kQ6_K, MODE, 4>(a, 1, s);
+            else if (!mgs_launch_t<kQ6_K, MODE>(a, 1, s)) mmx_launch<MODE, false>(g, s);
             break;
-        case kQ6_K:
-            if (g.qx != nullptr) {
-                MgArgs a{};
-                a.a = g;
-                a.m[0] = g.m; a.out[0] = g.out; a.ostride[0] = g.ostride; a.qx[0] = g.qx; a.qxd[0] = g.qxd;
-                if (!mgs_launch_t<kQ6_K, MODE>(a, 1, s)) mmx_launch<MODE, false>(g, s);
-                break;
-            }
-            if (kq_g == 4) hipLaunchKernelGGL((k_mmk<MODE, 4>), kq_grid, dim3(kThreads), 0, s, g);
-            else if (kq_g == 2) hipLaunchKernelGGL((k_mmk<MODE, 2>), kq_grid, dim3(kThreads), 0, s, g);
-            else hipLaunchKernelGGL((k_mmk<MODE, 1>), kq_grid, dim3(kThreads), 0, s, g);
-            break;
+        }
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -21,7 +21,7 @@ from test_gpu_kernels import BLOCK, Q4_0, Q4_1, Q4_K, Q5_0, Q6_K, Q8_0, Q8K, TQ2
 TYPES = (Q4_0, Q4_1, Q5_0, Q8_0, TQ2_0, Q4_K, Q6_K)
 # rows, values, tokens: short of a row group, of a workgroup, of a chunk; then enough workgroups for the wider token tiles
 SHAPES = [(1, 256, 2), (31, 512, 8), (33, 1024, 9), (129, 768, 31), (300, 256, 33), (1153, 512, 250), (2100, 512, 513),
-          (70, 2048, 8), (33, 2304, 9), (65, 4352, 7), (8161, 256, 3), (8193, 256, 3)]
+          (70, 2048, 8), (33, 2304, 9), (65, 4352, 7), (8161, 256, 3), (8193, 256, 3), (3001, 512, 190)]
 PARTIAL = [(40, 32, 3), (130, 288, 17), (65, 1120, 40), (1153, 288, 80), (1153, 1120, 250), (2100, 288, 513)]
 NOT_FINITE = [(70, 512, 20), (70, 512, 700), (1153, 512, 250), (2100, 512, 513)]  # shared chunks, then 8, 16 and 32 tokens
 

@@ -23,7 +23,7 @@ import pyoracle  # noqa: E402
 FORMATS = {"q4_0": G.T_Q4_0, "q4_1": G.T_Q4_1, "q5_0": G.T_Q5_0, "q8_0": G.T_Q8_0, "q4_k": G.T_Q4_K, "q5_k": G.T_Q5_K,
            "q6_k": G.T_Q6_K, "tq2_0": G.T_TQ2_0}
 SHAPES = {"ff": (512, 8, 2048), "embd": (2304, 4, 256)}  # hidden width, query heads, feed-forward width
-LENGTHS = (2, 5, 8, 16, 33, 64, 130, 200, 517)
+LENGTHS = (2, 5, 8, 16, 33, 64, 130, 200, 250, 517)
 VARIANTS = [(f, {}) for f in FORMATS] + [("q4_k", {"BRISK_HIP_PAIR_SPLIT": "1"}), ("q4_k", {"BRISK_HIP_PREFILL_Q4X": "1"}),
                                          ("q5_k", {"BRISK_HIP_PREFILL_MX": "0"}), ("q6_k", {"BRISK_HIP_PREFILL_MX": "0"})]
 
