@@ -2594,7 +2594,7 @@ __global__ __launch_bounds__(kThreads) void k_pre_attn_fa(PreAttnArgs p, int nto
 // launches: what each token's step needs that no other token's state enters (the conv, the norms, the
 // gates: every token at once), the delta rule itself (the one serial part), and the gated norm of its
 // outputs (every token at once again).  One workgroup a head that ran whole steps spent 6.2 us a token
-// on barriers, one-lane sums and 128 state rows in two waves; here the serial part is 0.89 us a token (16
+// on barriers, one-lane sums and 128 state rows in two waves; here the serial part is 0.87 us a token (16
 // heads of 128 x 128, 512 tokens: 3.2 ms a layer before, 0.5 now).
 
 // Normalised q and k, and v, of every token into p.conv ([token][3 heads DIM]); decay and beta into
@@ -2665,8 +2665,9 @@ __global__ __launch_bounds__(DIM) void k_pre_ssm_in(PreSsmArgs p) {
 // both sums sequential in i as the reference's.  A sum walks the row's lanes: at each of eight phases
 // every lane adds its terms to the running sum taken from the lane before it, and lane p's is the real
 // one after phase p.  The products are formed ahead of the sums, and o of the token before is summed
-// beside this token's first sum, so two chains of dependent adds share the issue slots.  Bound by those
-// chains: 2 x DIM adds a token.  The state halves are the decode step's (position p reads half p & 1):
+// beside this token's first sum, so two chains of dependent adds share the issue slots.  Bound by the one
+// wave's issue: some 470 instructions a token (DIM 128) at 4 cycles, 2 x DIM of them those adds, are 0.78 of its
+// 0.87 us.  The state halves are the decode step's (position p reads half p & 1):
 // the half of the last token's parity keeps the state before it (the reference's snapshot,
 // src/model.cpp:798-812), the other half the state after it.
 constexpr int kDppShr1 = 0x111;  // lane i takes lane i - 1's value (within 16 lanes)
@@ -2781,7 +2782,7 @@ __global__ __launch_bounds__(DIM) void k_pre_ssm_out(PreSsmArgs p) {
 
 // The expanded-plane GEMM: 4 waves (128 rows) a workgroup when that still gives every compute unit
 // two workgroups, else 2 waves, else 1.  At one wave a SIMD a CU holds four waves either way; smaller
-// workgroups couple fewer waves at each super-block's barrier (down on configs[2]: 59 us with 4
+// workgroups couple fewer waves at each super-block's barrier (2048 x 8192, 512 tokens: 59 us with 4
 // waves a workgroup, 50 with 2 or 1).
 template <int MODE, bool KM>
 static void mmx_launch(const MmArgs& g, hipStream_t s) {

@@ -1197,8 +1197,6 @@ void Session::validate(const int32_t* tokens, size_t n) const {
     if (n > max_ctx_ - position_) throw Error(BRISK_HIP_EINVAL, "model: context length exceeded");
 }
 
-// Writes tokens to seq[position_ ..], syncs the device position to the host's and
-// marks seq[0, position_ + n) as caller tokens (pos_[1]).
 // rows x vocab logits from the device into out (when given) through the pinned staging; waits for the stream.
 void Session::fetch_logits(float* out, const float* dev, size_t rows) {
     const size_t bytes = rows * static_cast<size_t>(cfg_.vocab) * 4;
@@ -1208,6 +1206,8 @@ void Session::fetch_logits(float* out, const float* dev, size_t rows) {
     if (out != nullptr) std::memcpy(out, hb, bytes);
 }
 
+// Writes tokens to seq[position_ ..], syncs the device position to the host's and
+// marks seq[0, position_ + n) as caller tokens (pos_[1]).
 void Session::stage(const int32_t* tokens, size_t n) { stage(tokens, n, position_); }
 
 void Session::stage(const int32_t* tokens, size_t n, size_t device_pos) {
@@ -1231,12 +1231,12 @@ bool Session::use_prefill(size_t n) const {
     const bool mfma_fits = prefill_mfma_ && pre_attn_mfma_fits(static_cast<int>(cfg_.heads / cfg_.kv_heads), static_cast<int>(cfg_.head_dim));
     // Gemma 3 (sliding layers, post-norms, GELU, soft-capped logits) and LFM2 (short convolutions)
     // take the exact attention only
-    // Qwen3.5: the projections batched, the recurrence over the tokens in one launch (state sizes 64
-    // and 128), the plain attention batched (contexts of its LDS window)
+    // Qwen3.5: the projections batched, the recurrence over the tokens in three launches (state sizes
+    // 64 and 128), the plain attention batched (contexts of its LDS window)
     if (qwen35())
         return prefill_on_ && n >= 2 && pre_ssm_fits(static_cast<int>(cfg_.ssm_state)) && pre_plain_fits(static_cast<int>(position_ + n));
-    // the plain attention batched (contexts of its LDS window); Gemma 4's per-layer shapes and
-    // per-layer embeddings take their prompts token by token
+    // the plain attention batched (contexts of its LDS window), Gemma 4's per-layer shapes and
+    // per-layer embeddings among them
     if (plain_attn_) return prefill_on_ && n >= 2 && pre_plain_fits(static_cast<int>(position_ + n));
     if (gemma() || lfm2()) return prefill_on_ && n >= 2 && exact_fits && cfg_.head_dim <= 128;
     return prefill_on_ && n >= 2 && (exact_fits || mfma_fits);
