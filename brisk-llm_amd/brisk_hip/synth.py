@@ -8,7 +8,7 @@ the ones the reference's loader reads (src/model.cpp:161-301, :303-423): GGUF
 dims innermost first, so a rows x cols matrix is stored as {cols, rows}
 (src/model.cpp:462).
 
-Distributions (where a config leaves a scale open it is
+Distributions (the workloads'; where one leaves a scale open it is
 pinned here so activations stay O(1) through the layers):
   Q4_0  d = half(U(0.001, 0.02)), nibbles uniform 0..15
   Q8_0  d = half(U(0.0002, 0.004)), values uniform -127..127
@@ -217,15 +217,15 @@ def _uniform4(t):
 
 
 SPECS = {
-    # configs[1]: Qwen3-0.6B shape, Q4_0 layers, Q8_0 embeddings and output.
+    # Qwen3-0.6B shape, Q4_0 layers, Q8_0 embeddings and output.
     "qwen3-0.6b": ModelSpec("qwen3-0.6b", "qwen3", 1024, 28, 16, 8, 128, 3072, 151936, 1e6, fmt=_uniform4(G.T_Q4_0)),
-    # configs[2]: Llama-3.2-1B shape in a Q4_K_M mix; tied Q6_K embedding.
+    # Llama-3.2-1B shape in a Q4_K_M mix; tied Q6_K embedding.
     "llama-3.2-1b": ModelSpec("llama-3.2-1b", "llama", 2048, 16, 32, 8, 64, 8192, 128256, 5e5, eps=1e-5, context=131072,
                               fmt={**_uniform4(G.T_Q4_K), "v": G.T_Q6_K, "down": G.T_Q6_K},
                               embd_fmt=G.T_Q6_K, out_fmt=None),
-    # configs[3]: Qwen3-1.7B shape, all Q8_0.
+    # Qwen3-1.7B shape, all Q8_0.
     "qwen3-1.7b": ModelSpec("qwen3-1.7b", "qwen3", 2048, 28, 16, 8, 128, 6144, 151936, 1e6, fmt=_uniform4(G.T_Q8_0)),
-    # configs[4]: BitNet b1.58 2B4T shape, TQ2_0 layers; tied Q4_0 embedding.
+    # BitNet b1.58 2B4T shape, TQ2_0 layers; tied Q4_0 embedding.
     "bitnet-2b": ModelSpec("bitnet-2b", "bitnet-b1.58", 2560, 30, 20, 5, 128, 6912, 128256, 5e5, eps=1e-5, context=4096,
                            fmt=_uniform4(G.T_TQ2_0), embd_fmt=G.T_Q4_0, out_fmt=None),
     # Small shapes of each family for the parity tests (the oracle finishes them in well under a second).

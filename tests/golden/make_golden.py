@@ -30,9 +30,9 @@ import pyoracle  # noqa: E402
 
 # name -> (prompt length, greedy steps)
 RUNS = {
-    "qwen3-0.6b": (32, 256),      # configs[1]
-    "bitnet-2b": (64, 64),        # configs[4] (first 64 of its 256 steps)
-    "llama-3.2-1b": (64, 32),     # configs[2] shape, shorter prompt
+    "qwen3-0.6b": (32, 256),
+    "bitnet-2b": (64, 64),        # the first 64 of its 256 steps
+    "llama-3.2-1b": (64, 32),     # shorter prompt
     "tiny-qwen3": (12, 48),
     "tiny-llama": (12, 48),
     "tiny-q8": (12, 48),
@@ -62,9 +62,9 @@ def logit_sample(logits):
 # Each step stores the reference's top 8 logits and a strided sample (every `stride`-th entry), so the GPU
 # session's logits can be held to the tolerance at every step, not only at the prompt.
 STEP_RUNS = {
-    "qwen3-0.6b": (32, 7, 256),       # configs[1]
-    "llama-3.2-1b": (512, 11, 128),   # configs[2]: 512-id prefill, then 128 greedy steps
-    "bitnet-2b": (64, 7, 256),        # configs[4]
+    "qwen3-0.6b": (32, 7, 256),
+    "llama-3.2-1b": (512, 11, 128),   # 512-id prefill, then 128 greedy steps
+    "bitnet-2b": (64, 7, 256),
 }
 SAMPLE_POINTS = 32
 
@@ -105,7 +105,7 @@ def steps_fixture(name):
 
 
 def long_context_fixture(n_pos=4096, n_gen=128, kv_seed=7, token=11):
-    """configs[3]: Qwen3-1.7B-shape Q8_0 with every layer's K and V cache pre-filled to n_pos positions
+    """Qwen3-1.7B-shape Q8_0 with every layer's K and V cache pre-filled to n_pos positions
     with seeded fp16 N(0,1) values (numpy default_rng(kv_seed), layer by layer, key then value), then
     greedy steps from `token`.  Run by the oracle (the C restatement, which takes a pre-filled cache)."""
     from brisk_hip import model
@@ -157,7 +157,7 @@ if __name__ == "__main__":
     if args and args[0] == "steps":        # make_golden.py steps [names...]: the per-step fixtures
         for n in args[1:] or list(STEP_RUNS):
             steps_fixture(n)
-    elif args and args[0] == "long":       # make_golden.py long: configs[3] on the pre-filled cache
+    elif args and args[0] == "long":       # make_golden.py long: Qwen3-1.7B shape on the pre-filled cache
         long_context_fixture()
     else:
         main(args or list(RUNS))

@@ -3,7 +3,7 @@ made from the reference's own Model(file, repack = false) and driven the way the
 drives an Engine (oracle/hip_engine_shim.cpp, built into oracle/_ref/libhip_engine.so):
 
   - cmd_generate's greedy loop over Engine::eval (src/main.cpp:287-299) and the on-device
-    generate_greedy fast path: configs[1]'s 256 ids equal the reference Session's (the golden
+    generate_greedy fast path: the Qwen3-0.6B shape's 256 ids equal the reference Session's (the golden
     fixture), and every family's tiny model gives the reference's ids and prompt logits;
   - cmd_generate --draft (src/main.cpp:236-276): the reference's Speculator over the HipSession
     target, with the lookup drafter and with a CPU ModelDrafter, settles exactly the greedy ids;

@@ -1,9 +1,9 @@
 """Every benchmark config's full workload against reference-written fixtures, with the
-logits held to the north-star tolerance (max-abs 2e-2) at every step.
+logits held to max-abs 2e-2 at every step.
 
 tests/golden/*_steps.json were written by tests/golden/make_golden.py: the reference's
-CPU engine (oracle/_ref) for configs[1], [2] and [4]; the oracle (oracle/oracle.c, pinned
-to oracle/_ref) for configs[3], whose K/V caches are pre-filled with seeded fp16 N(0,1)
+CPU engine (oracle/_ref) for the Qwen3-0.6B, Llama and BitNet shapes; the oracle (oracle/oracle.c, pinned
+to oracle/_ref) for the Qwen3-1.7B shape, whose K/V caches are pre-filled with seeded fp16 N(0,1)
 values.  Each step holds the greedy pick, the top 8 logits and a strided sample.
 
 Two checks a config: the session's own greedy run (prompt, then one persistent-loop
@@ -75,7 +75,7 @@ def _h2d(dst_ptr, host, nbytes):
 
 
 def test_config3_long_context():
-    """configs[3]: Qwen3-1.7B-shape Q8_0, K/V pre-filled to 4096 positions (the fixture's seeded values,
+    """Qwen3-1.7B-shape Q8_0, K/V pre-filled to 4096 positions (the fixture's seeded values,
     regenerated here layer by layer, key then value), then the fixture's greedy steps (the loop's
     exact spread attention)."""
     g = fixture("qwen3-1.7b_kv4096_steps.json")

@@ -1,5 +1,5 @@
-"""Long contexts: KV caches pre-filled with seeded fp16 N(0,1) values (as configs[3]
-does to 4096 positions), then decode, against the oracle running on the same
+"""Long contexts: KV caches pre-filled with seeded fp16 N(0,1) values (to
+4096 positions at full size), then decode, against the oracle running on the same
 pre-filled cache (brisk_hip_session_kv_cache / set_position on the GPU,
 or_session_kv / set_position in the oracle).
 
@@ -11,7 +11,7 @@ loop attention takes whole (more than 4 query heads a kv head, partial rotary,
 or heads-per-kv x length beyond the spread attention's 16384 scores, as
 Llama-3.2-1B beyond 4096 positions) runs on the one-kernel-per-phase path.  So
 the tiny models' logits are bit-identical to the oracle's, and the full-size
-case is held step by step to the north-star tolerance (max-abs 2e-2) with
+case is held step by step to the tolerance (max-abs 2e-2) with
 identical greedy ids.
 """
 import numpy as np
@@ -117,7 +117,7 @@ def test_plain_attention_value_batches(name):
 
 @pytest.mark.slow
 def test_qwen3_1_7b_at_4096():
-    """configs[3] at full size: Qwen3-1.7B-shape Q8_0, 4096 pre-filled positions, then decode."""
+    """Full size: Qwen3-1.7B-shape Q8_0, 4096 pre-filled positions, then decode."""
     f, cfg, table = model.load(synth.model_path("qwen3-1.7b"))
     n_pos = 4096
     print(f"[long] qwen3-1.7b: KV pre-filled to {n_pos}", flush=True)

@@ -10,11 +10,11 @@ Opt-in path (BRISK_HIP_PREFILL_ATTN=mfma): from 64 tokens on, the causal
 attention runs flash style on v_mfma_f32_16x16x32_f16 with hi/lo f16 operands
 (fp32 rounding of each product, not the reference's summation order).  Its
 reordering can tip an int8 re-quantisation downstream, after which later layers
-differ by a quantisation step: on configs[2] at 512 tokens the logits move by
-about 0.03, beyond the north-star 2e-2, which is why it is not the default.  Its
+differ by a quantisation step: on the Llama-3.2-1B shape at 512 tokens the logits move
+by about 0.03, beyond the 2e-2 that every path is held to, which is why it is not the default.  Its
 tests pin what it does guarantee: on tiny models most prompts give the oracle's
 logits to the bit and none moves by more than a few quantisation steps; on
-configs[2] the greedy pick is the reference's and the logits stay within 0.1.
+that shape the greedy pick is the reference's and the logits stay within 0.1.
 """
 import os
 
@@ -90,7 +90,7 @@ def test_mfma_attention_tiny(name):
 @pytest.mark.slow
 @pytest.mark.skipif(not pyoracle.ref_available(), reason="oracle/_ref/libbrisk_ref.so is not built (no reference tree)")
 def test_mfma_attention_llama_512():
-    """configs[2] (Llama-3.2-1B-shape Q4_K_M), 512-token prompt against the
+    """Llama-3.2-1B shape, Q4_K_M, 512-token prompt against the
     reference engine: the default path bit for bit, the opt-in MFMA attention
     with the same greedy pick and logits within 0.1."""
     path = synth.model_path("llama-3.2-1b")

@@ -1,7 +1,7 @@
 """GPU parity of the HIP session (Engine counterpart) against the oracle.
 
 Tiny models of each family the benchmark configs use, seeded: prompt logits
-within 2e-2 (fp32 accumulation-order tolerance of the north star), greedy ids
+within 2e-2 (fp32 accumulation-order tolerance), greedy ids
 identical, eval_all rows, rollback, and the reference's error messages.
 """
 import os

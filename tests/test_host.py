@@ -81,7 +81,7 @@ def test_synthetic_blocks_are_deterministic_and_in_range():
     a, b = synth.q4_0_blocks(9, 100), synth.q4_0_blocks(9, 100)
     assert np.array_equal(a, b)
     d = a[:, 0:2].copy().view(np.float16).astype(np.float32)
-    assert np.all((d >= 0.0009) & (d <= 0.0201))  # configs[0]: d ~ U(0.001, 0.02)
+    assert np.all((d >= 0.0009) & (d <= 0.0201))  # d ~ U(0.001, 0.02)
     q8 = synth.q8_0_blocks(9, 100)
     assert np.all(q8[:, 2:].view(np.int8) >= -127)
     t = synth.tq2_0_blocks(9, 10)
@@ -90,7 +90,7 @@ def test_synthetic_blocks_are_deterministic_and_in_range():
 
 
 def test_spec_bytes_match_the_measurement_contract():
-    """decode bytes of configs[1] (Qwen3-0.6B Q4_0 + Q8_0 output) at position 0."""
+    """decode bytes of the Qwen3-0.6B shape (Q4_0 + Q8_0 output) at position 0."""
     s = synth.SPECS["qwen3-0.6b"]
     assert s.layers * s.layer_weight_bytes() == 247_726_080
     assert s.output_bytes() == 165_306_368

@@ -451,7 +451,7 @@ def test_oracle_greedy_matches_reference_fixture(name):
 
 
 def test_oracle_first_tokens_of_qwen3_0_6b_fixture():
-    """configs[1] at full size: the first greedy ids of the reference's 256-step run."""
+    """Qwen3-0.6B shape at full size: the first greedy ids of the reference's 256-step run."""
     with open(os.path.join(HERE, "golden", "qwen3-0.6b_greedy.json")) as fh:
         g = json.load(fh)
     path, f, cfg, table = tiny("qwen3-0.6b")
